@@ -1425,20 +1425,58 @@ void kp_stage_z(const PersistDev P, const Real a, const Real b, const int fold, 
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-static int pick_chunk(const int nd, const int64_t columns, const int mult)
+// march length of a launch that shares the chip: a slab of a pipelined step
+// (the other stream's sweep fills its tail) and the split x / y sweeps
+static int pick_chunk(const int nd, const int64_t columns)
 {
-    // enough marching threads for ~4 waves per SIMD (256 CUs x 4 SIMDs), times
-    // mult: a launch that runs alone wants more (its sweeps hold two waves per
-    // SIMD, and the last partial round of waves otherwise idles most of the
-    // chip); a slab of a pipelined step shares the chip with the other
-    // stream's sweep, which fills that tail
-    const int64_t target_threads = 256LL * 4 * 4 * 64 * mult;
+    // enough marching threads for ~4 waves per SIMD (256 CUs x 4 SIMDs)
+    const int64_t target_threads = 256LL * 4 * 4 * 64;
     int nchunks = (int)((target_threads + columns - 1) / columns);
     if (nchunks < 1) nchunks = 1;
     int chunk = (nd + nchunks - 1) / nchunks;
     if (chunk < 16) chunk = nd < 16 ? nd : 16;
     return chunk;
 }
+
+// March length of a fused x+y (dir 3) or z (dir 2) sweep launch that runs
+// alone: the one with the least modelled time.  `blocks` four-wave workgroups
+// cover the marching columns; cut into chunks of L rows, the busiest of the
+// 256 CUs runs n = ceil(blocks * chunks / 256) of them, two at a time, and a
+// chunk costs its rows plus `ov` rows of start-up (window fill and the rows
+// whose flux is recomputed at the chunk's first face; for the z sweep also
+// the five extra rows of u it reads).  `lat` rows pass once per launch before
+// the first row is done.  A workgroup alone on its CU takes 1.2 times its
+// share.  Measured on MI355X over L = 1..64 for blocks from 16^3 to 192^3, the
+// model is within 10 % in every arithmetic build.  Chunks of at least 16 rows
+// (four waves per SIMD and more) left small blocks to a few dozen waves
+// marching 16 rows each: FAST x+y / z sweep 42 / 27 us at 32^3, 45 / 29 at
+// 64^3 and 100 / 54 at 128^3, against 9 / 10, 22 / 17 and 96 / 53 here.
+static int whole_march(const int nd, const int64_t blocks, const int dir)
+{
+    const double lat = dir == 3 ? 3.0 : 1.0;
+    const double ov = dir == 3 ? 1.0 : kFast ? 3.0 : 2.0;
+    int best = nd;
+    double least = 0.0;
+    for (int L = nd; L >= 1;) {
+        const int nch = (nd + L - 1) / L;
+        const int64_t n = (blocks * nch + 255) / 256;
+        if (L < nd && n > 64) break;     // the tail no longer matters
+        const double t = lat + (n == 1 ? 1.2 : (double)n) * (L + ov);
+        if (L == nd || t < least) { least = t; best = L; }
+        const int next = (nd + nch) / (nch + 1);   // the longest march with more chunks
+        L = next < L ? next : L - 1;
+    }
+    return best;
+}
+
+// four-wave workgroups of one chunk of the x+y sweep over nz planes / of the
+// z sweep's flattened (x, y) columns
+static int xy_blocks(const Geom& g, const int nz)
+{
+    const int waves = ((g.nx + 6) * nz + XY_TILE - 1) / XY_TILE;
+    return (waves + 3) / 4;
+}
+static int z_blocks(const Geom& g) { return (g.nx * g.ny + 255) / 256; }
 
 static int rows_grid(const Geom& g)
 {
@@ -1515,28 +1553,27 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
     A.sos_next = p.sos_next; A.sos_cpu = p.sos_cpu;
     A.z0 = p.z0; A.z1 = p.z1 < 0 ? g.nz : p.z1;
     const int nzr = A.z1 - A.z0;
-    // a whole-block launch (not a slab) targets four times a slab's waves:
-    // at 256^3-512^3 its steps are 0.6-2.7 % faster than with twice
-    const int alone = (A.z0 == 0 && A.z1 == g.nz) ? 4 : 1;
+    const bool whole = A.z0 == 0 && A.z1 == g.nz;   // not a slab
     if (dir == 3) {
-        const int chunk = pick_chunk(g.ny, (int64_t)g.nx * nzr, alone);
-        const int waves = ((g.nx + 6) * nzr + XY_TILE - 1) / XY_TILE;
-        const dim3 grid((waves + 3) / 4, (g.ny + chunk - 1) / chunk);
+        const int nb = xy_blocks(g, nzr);
+        const int chunk = whole ? whole_march(g.ny, nb, 3) : pick_chunk(g.ny, (int64_t)g.nx * nzr);
+        const dim3 grid(nb, (g.ny + chunk - 1) / chunk);
         // a first stage of a folded build does not read R
         if (kFold && A.a == Real(0.0f)) hipLaunchKernelGGL(k_sweep_xy<true>, grid, dim3(64, 4), 0, s, g, A, chunk);
         else                            hipLaunchKernelGGL(k_sweep_xy<false>, grid, dim3(64, 4), 0, s, g, A, chunk);
     } else if (dir == 0) {
         const int npen = g.ny * nzr;
-        const int chunk = pick_chunk(g.nx, npen, 1);
+        const int chunk = pick_chunk(g.nx, npen);
         dim3 grid((npen + 63) / 64, (g.nx + chunk - 1) / chunk);
         hipLaunchKernelGGL(k_sweep_x, grid, dim3(64), 0, s, g, A, chunk);
     } else if (dir == 1) {
-        const int chunk = pick_chunk(g.ny, (int64_t)g.nx * nzr, 1);
+        const int chunk = pick_chunk(g.ny, (int64_t)g.nx * nzr);
         dim3 grid((g.nx * nzr + 255) / 256, (g.ny + chunk - 1) / chunk);
         hipLaunchKernelGGL((k_sweep_yz<1, MODE_ACC>), grid, dim3(256), 0, s, g, A, chunk);
     } else {
-        const int chunk = pick_chunk(nzr, (int64_t)g.nx * g.ny, alone);
-        const dim3 grid((g.nx * g.ny + 255) / 256, (nzr + chunk - 1) / chunk);
+        const int nb = z_blocks(g);
+        const int chunk = whole ? whole_march(nzr, nb, 2) : pick_chunk(nzr, (int64_t)g.nx * g.ny);
+        const dim3 grid(nb, (nzr + chunk - 1) / chunk);
         if (stage == 2)      hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE_NOR>), grid, dim3(256), 0, s, g, A, chunk);
         else if (stage == 1) hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE>), grid, dim3(256), 0, s, g, A, chunk);
         else                 hipLaunchKernelGGL((k_sweep_yz<2, MODE_CONV>), grid, dim3(256), 0, s, g, A, chunk);
@@ -1605,22 +1642,23 @@ void launch_test_face(const int n, const int dir, const void* stv, void* outv, h
     else               hipLaunchKernelGGL(k_test_face<2>, grid, block, 0, s, n, st, out);
 }
 
-int default_chunk(const int nd, const long long columns) { return pick_chunk(nd, columns, 1); }
-// the march length of a whole-block launch that runs alone
-int whole_chunk(const int nd, const long long columns) { return pick_chunk(nd, columns, 4); }
+// the march length of a whole-block x+y (dir 3) or z (dir 2) launch that runs alone
+int whole_chunk(const Geom& g, const int dir)
+{
+    return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3) : whole_march(g.nz, z_blocks(g), 2);
+}
 
 // grid of the fused x+y sweep: dims[0] blocks of four waves over the padded
 // rows of all planes, dims[2] y-chunks (dims[1] = 1)
 void xy_grid(const Geom& g, const int chunk, int dims[3])
 {
-    const int waves = ((g.nx + 6) * g.nz + XY_TILE - 1) / XY_TILE;
-    dims[0] = (waves + 3) / 4; dims[1] = 1; dims[2] = (g.ny + chunk - 1) / chunk;
+    dims[0] = xy_blocks(g, g.nz); dims[1] = 1; dims[2] = (g.ny + chunk - 1) / chunk;
 }
 
 // grid of the z sweep: dims[0] blocks of 256 flattened (x, y) columns, dims[2] z-chunks
 void z_grid(const Geom& g, const int chunk, int dims[3])
 {
-    dims[0] = (g.nx * g.ny + 255) / 256; dims[1] = 1; dims[2] = (g.nz + chunk - 1) / chunk;
+    dims[0] = z_blocks(g); dims[1] = 1; dims[2] = (g.nz + chunk - 1) / chunk;
 }
 
 void batch_sos(const BatchDev& B, const int blocks, const int cpu_form, const double cfl, const double dt_max,

@@ -120,8 +120,7 @@ void persist_stage(const PersistDev& P, const int blocks[2], int threads, double
 int persist_occupancy(int threads, int phase);                                                             \
 void xy_grid(const Geom& g, int chunk, int dims[3]);                                                       \
 void z_grid(const Geom& g, int chunk, int dims[3]);                                                        \
-int default_chunk(int nd, long long columns);                                                              \
-int whole_chunk(int nd, long long columns);                                                                \
+int whole_chunk(const Geom& g, int dir);                                                                   \
 } }
 
 MPCF_DECLARE_LAUNCHERS(parity)

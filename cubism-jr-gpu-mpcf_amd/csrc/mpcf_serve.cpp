@@ -514,9 +514,9 @@ bool rebuild(mpcf_server* S)
         // a lone case marches as a whole-block single-case launch would
         // (shorter chunks, more waves to fill the chip); a mix shares the
         // chip and takes the longer, cheaper chunks of adaptive_march
-        const int lxy = n == 1 ? mpcf::parity::whole_chunk(c->g.ny, (long long)c->g.nx * c->g.nz)
+        const int lxy = n == 1 ? mpcf::fast::whole_chunk(c->g, 3)
                                : mpcf::detail::adaptive_march(c->g.ny, cols_xy);
-        const int lz = n == 1 ? mpcf::parity::whole_chunk(c->g.nz, (long long)c->g.nx * c->g.ny)
+        const int lz = n == 1 ? mpcf::fast::whole_chunk(c->g, 2)
                               : mpcf::detail::adaptive_march(c->g.nz, cols_z);
         mpcf::detail::case_desc(c, c->cur, lxy, lz, hc[i], blocks);
         oxy[j + 1] = oxy[j] + blocks[0];
