@@ -61,6 +61,14 @@ inline Geom make_geom(int nx, int ny, int nz)
     return g;
 }
 
+// the longest z march: the z sweep addresses the rows of a chunk by 32-bit byte
+// offsets from its first row (binary64 storage, less two planes for the lanes)
+inline int z_march_limit(const Geom& g)
+{
+    const int64_t rows = (int64_t(1) << 32) / ((int64_t)g.px * g.py * 8) - 2;
+    return rows < 1 ? 1 : rows > g.nz ? g.nz : (int)rows;
+}
+
 // device-resident step state: the max speed of sound of the last reduction,
 // the time step derived from it and the dt/h every stage reads.  The
 // reduction targets and counters must be zero when a block is created.  Builds whose

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -226,7 +227,7 @@ inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const 
     d.u[0] = c->u[0]; d.u[1] = c->u[1]; d.R = c->R; d.acc = c->acc; d.st = c->st; d.h = c->h;
     for (int f = 0; f < 6; ++f) d.bc[f] = c->bc[f];
     d.chunk_xy = len_xy;
-    d.chunk_z = len_z;
+    d.chunk_z = std::min(len_z, z_march_limit(c->g));
     int dims[3];
     parity::xy_grid(c->g, d.chunk_xy, dims);
     d.nbx_xy = dims[0]; d.nby_xy = dims[1];

@@ -18,6 +18,7 @@
 // Accumulators carry the partial flux sums between sweeps in the reference's
 // summation order (((((fxp-fxm)+fyp)-fym)+fzp)-fzm) (GPUkernels.cu:1111).
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <type_traits>
 #include "mpcf_scheme.h"
 #include "mpcf_launch.h"
@@ -180,40 +181,56 @@ __device__ __forceinline__ int bc_index(const int i, const int n, const int bcma
 }
 
 // A lane's element index split into a part that is the same for every lane of
-// the wave (base, a scalar) and the lane's byte offset from it (lo, small and
-// non-negative).  The fused x+y sweep accesses its fields through buffer
-// resources built on wave-uniform element pointers (the field, row and wave
-// parts of the index, added by the scalar unit), with the lane's 32-bit
-// offset: as flat global accesses the same loads and stores took one 64-bit
-// vector add each, 3 % of its vector instructions.  The y and z sweeps use the
-// same split with flat global accesses (see ld_lane).
+// the wave (base, a scalar: the element of a row the march starts from) and
+// the lane's byte offset from it (lo, small and non-negative).
+// An access is a global load or store of a scalar base and a 32-bit vector
+// offset, `ld_lane(p, off)`: the sweeps keep one scalar base per field for the
+// whole march and add the row's bytes to the lane's offset, one vector add
+// that all fields of the row share.  Buffer resources rebuilt per access took
+// 165 scalar instructions a row in the x+y sweep (30 now), 64-bit flat
+// addresses 29 64-bit vector adds a row in the z sweep (none now; its E-pair
+// instance fits two waves per SIMD again).  100 steps of 128^3 with transfers
+// 44.2 -> 43.6 ms, 30 steps of 512^3 661 -> 656 ms.
 struct LaneIdx { int64_t base; uint32_t lo; };
 
 // e: the lane's element; floor_e: an element no greater than the element of
-// any active lane of the wave (the first active lane's value is taken)
-__device__ __forceinline__ LaneIdx lane_idx(const int e, const int floor_e)
+// any active lane of the wave (the first active lane's value is taken);
+// shift: wave-uniform elements from there to the row the march starts from
+__device__ __forceinline__ LaneIdx lane_idx(const int e, const int floor_e, const int64_t shift)
 {
     const int b = __builtin_amdgcn_readfirstlane(floor_e);
-    return LaneIdx{b, (uint32_t)(e - b) * (uint32_t)sizeof(Real)};
+    return LaneIdx{b + shift, (uint32_t)(e - b) * (uint32_t)sizeof(Real)};
 }
 
-// raw buffer resource at a wave-uniform address: no stride, no record limit,
-// 32-bit data format (a zero format would read as zero)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_at(const void* p)
+// wave-uniform pointers of the first N fields at p, fs elements apart, each in
+// a scalar register pair of its own: hidden from the optimizer, which would
+// otherwise add the lane offset once and then every field's distance with a
+// 64-bit vector add
+#define MPCF_GLOBAL __attribute__((address_space(1)))
+template <int N, typename V> struct Bases
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, -1, 0x00020000);
-}
+    V MPCF_GLOBAL* p[N];
+    __device__ __forceinline__ Bases(V* const p0, const int64_t fs)
+    {
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            // uniform by construction; a pointer read from a table in memory may
+            // sit in a vector register
+            const uint64_t a = (uint64_t)(p0 + q * fs);
+            const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+            const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+            uint64_t b = ((uint64_t)hi << 32) | lo;
+            asm("" : "+s"(b));
+            p[q] = (V MPCF_GLOBAL*)b;
+        }
+    }
+};
 
-// element p[u] + lane offset lo (u wave-uniform).  BUF: through a buffer
-// resource; else a flat global access (the y/z sweeps: their marches keep
-// more scalar state live, and a resource per access runs them out of scalar
-// registers)
-template <bool BUF, typename V>
-__device__ __forceinline__ V ld_lane(const V* p, const int64_t u, const uint32_t lo)
+// the element `off` bytes after the wave-uniform pointer p
+template <typename V>
+__device__ __forceinline__ V ld_lane(const V MPCF_GLOBAL* p, const uint32_t off)
 {
-    if constexpr (!BUF) return p[u + lo / sizeof(V)];
-    else if constexpr (sizeof(V) == 4) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rsrc_at(p + u), lo, 0, 0));
-    else return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc_at(p + u), lo, 0, 0));
+    return *(const V MPCF_GLOBAL*)((const char MPCF_GLOBAL*)p + off);
 }
 
 // store; STREAM: non-temporal, for data that no kernel reads again soon --
@@ -222,32 +239,45 @@ __device__ __forceinline__ V ld_lane(const V* p, const int64_t u, const uint32_t
 // the z sweep of the slab).  The hint keeps these streams from displacing
 // lines in the caches; at 512^3 it takes the pipelined step from 20.66 to
 // 20.0 ms.
-template <bool BUF, bool STREAM = false, typename V>
-__device__ __forceinline__ void st_lane(V* p, const int64_t u, const uint32_t lo, const V v)
+template <bool STREAM = false, typename V>
+__device__ __forceinline__ void st_lane(V MPCF_GLOBAL* p, uint32_t off, const V v)
 {
-    constexpr int aux = STREAM ? 2 : 0;   // bit 1: nt
-    if constexpr (!BUF) {
-        if (STREAM) __builtin_nontemporal_store(v, &p[u + lo / sizeof(V)]);
-        else        p[u + lo / sizeof(V)] = v;
-    } else if constexpr (sizeof(V) == 4)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc_at(p + u), lo, 0, aux);
-    else
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v),
-                                              rsrc_at(p + u), lo, 0, aux);
+    // the address is formed here, not shared with a load of the same element:
+    // across a branch it would be kept as a 64-bit vector sum
+    asm("" : "+v"(off));
+    V MPCF_GLOBAL* const q = (V MPCF_GLOBAL*)((char MPCF_GLOBAL*)p + off);
+    if (STREAM) __builtin_nontemporal_store(v, q);
+    else        *q = v;
 }
 
-// raw conserved values of the cell at index `row` of a marched column (L =
-// element of row 0, s = element stride of the axis), boundary-mapped.  Returns
-// the sign the axis' normal momentum takes; the caller applies it where the
-// values are consumed, so that a prefetch is not waited on when it is issued.
-template <bool BUF>
-__device__ __forceinline__ Real load_row(const StageArgs& A, const LaneIdx& L, const int row, const int n, const int s,
-                                         const int face_lo, Real* out)
+// raw conserved values of the cell at index `row` of a marched column, boundary-
+// mapped: U.p[q] + the lane's byte offset lo is field q's element of row r0, s
+// the element stride of the axis.  Returns the sign the axis' normal momentum
+// takes; the caller applies it where the values are consumed, so that a
+// prefetch is not waited on when it is issued.
+__device__ __forceinline__ Real load_row(const StageArgs& A, const Bases<NU, const Real>& U, const uint32_t lo, const int r0,
+                                         const int row, const int n, const int s, const int face_lo, Real* out)
 {
     Real sg;
-    const int r = bc_index(row, n, A.bcmask, face_lo, sg);
+    const int r = bc_index(row, n, A.bcmask, face_lo, sg) - r0;
+    const uint32_t off = lo + (uint32_t)(r * s) * (uint32_t)sizeof(Real);
 #pragma unroll
-    for (int q = 0; q < NU; ++q) out[q] = ld_lane<BUF>(A.u, L.base + q*A.fs + (int64_t)r * s, L.lo);
+    for (int q = 0; q < NU; ++q) out[q] = ld_lane(U.p[q], off);
+    return sg;
+}
+// the same for the z axis, whose rows may lie further apart than 32-bit offsets
+// reach (the planes of the largest blocks): u0 + lo is field 0's element of
+// row r0, and the row's distance goes into the scalar pointers
+__device__ __forceinline__ Real load_row_far(const StageArgs& A, const Real* u0, const uint32_t lo, const int r0,
+                                             const int row, const int n, const int s, const int face_lo, Real* out)
+{
+    Real sg;
+    const int r = bc_index(row, n, A.bcmask, face_lo, sg) - r0;
+    const Bases<NU, const Real> U(u0 + (int64_t)r * s, A.fs);
+    uint32_t off = lo;
+    asm volatile("" : "+v"(off));   // kept 32-bit: widened once before the loop it would be a vector add per field
+#pragma unroll
+    for (int q = 0; q < NU; ++q) out[q] = ld_lane(U.p[q], off);
     return sg;
 }
 
@@ -266,56 +296,65 @@ struct EmitIn
     Real u[NU];
 };
 
+// fields of a y / z sweep at the march's first row, as wave-uniform pointers
 template <int MODE>
-__device__ __forceinline__ void emit_load(const StageArgs& A, const LaneIdx& L, const int64_t row, EmitIn<MODE>& in)
+struct EmitPtr
 {
-    const int64_t fs = A.fs;
-    const int64_t e = L.base + row;   // the wave-uniform part of the cell's element
-    if (MODE == MODE_FIRST) return;
-    if (!kFold || MODE == MODE_ACC) {
+    static constexpr bool kR = MODE == MODE_CONV || is_stage(MODE) || (kFold && MODE == MODE_ACC);
+    static constexpr bool kAll = MODE == MODE_FIRST || MODE == MODE_ACC || !kFold;   // all accumulators
+    Bases<kAll ? A_SUMG : 1, Real> acc;
+    Bases<3, Real> gp;                     // the G/P accumulators
+    Bases<kR ? NVAR : 1, Real> R;
+    Bases<is_stage(MODE) ? NU : 1, Real> uo;
+    __device__ __forceinline__ EmitPtr(const StageArgs& A, const int64_t base)
+        : acc(A.acc + base, A.fs), gp(A.acc + base + A_SUMG * A.fs, A.fs), R(A.R + base, A.fs), uo(A.uo + base, A.fs) {}
+};
+
+template <int MODE>
+__device__ __forceinline__ void emit_load(const EmitPtr<MODE>& E, const uint32_t off, EmitIn<MODE>& in)
+{
+    if constexpr (MODE != MODE_FIRST) {
+        if constexpr (EmitPtr<MODE>::kAll) {
 #pragma unroll
-        for (int q = 0; q < NACC; ++q) in.acc[q] = ld_lane<false>(A.acc, q*fs + e, L.lo);
-    } else {
+            for (int q = 0; q < NVAR; ++q) in.acc[q] = ld_lane(E.acc.p[q], off);
+        }
         // folded: only the G/P accumulators remain
-        in.acc[A_SUMG] = ld_lane<false>(A.acc, A_SUMG*fs + e, L.lo);
-        in.acc[A_SUMP] = ld_lane<false>(A.acc, A_SUMP*fs + e, L.lo);
-        in.acc[A_DIVU] = ld_lane<false>(A.acc, A_DIVU*fs + e, L.lo);
-    }
-    if (MODE == MODE_CONV || is_stage(MODE) || (kFold && MODE == MODE_ACC)) {
 #pragma unroll
-        for (int q = 0; q < NVAR; ++q) in.R[q] = ld_lane<false>(A.R, q*fs + e, L.lo);
+        for (int q = 0; q < 3; ++q) in.acc[A_SUMG + q] = ld_lane(E.gp.p[q], off);
+        if constexpr (EmitPtr<MODE>::kR) {
+#pragma unroll
+            for (int q = 0; q < NVAR; ++q) in.R[q] = ld_lane(E.R.p[q], off);
+        }
     }
 }
 
-// write the contribution of one cell.  F = flux at the cell's right face,
-// Fl = flux at its left face; cG/cP = plus-state + minus-state of G/P.
+// write the contribution of one cell, at byte offset `off` from the first
+// row of each field.  F = flux at the cell's right face, Fl = flux at its left
+// face; cG/cP = plus-state + minus-state of G/P.
 template <int MODE>
-__device__ __forceinline__ void emit(const StageArgs& A, const Real dtinvh, const LaneIdx& L, const int64_t row, const EmitIn<MODE>& in,
+__device__ __forceinline__ void emit(const StageArgs& A, const EmitPtr<MODE>& E, const Real dtinvh, const uint32_t off,
+                                     const EmitIn<MODE>& in,
                                      const FaceFlux& F, const FaceFlux& Fl, const Real cG, const Real cP,
                                      SosT& smax, bool& bad)
 {
-    Real* __restrict__ acc = A.acc;
-    const int64_t fs = A.fs;
-    const int64_t e = L.base + row;   // the wave-uniform part of the cell's element
-    const uint32_t lo = L.lo;
-    if (MODE == MODE_FIRST) {
+    if constexpr (MODE == MODE_FIRST) {
         // _xflux + _xextraterm_hllc ("=" assignment, GPUkernels.cu:57-59)
 #pragma unroll
-        for (int q = 0; q < NVAR; ++q) st_lane<false>(acc, q*fs + e, lo, F.f[q] - Fl.f[q]);
-        st_lane<false>(acc, A_SUMG*fs + e, lo, cG);
-        st_lane<false>(acc, A_SUMP*fs + e, lo, cP);
-        st_lane<false>(acc, A_DIVU*fs + e, lo, F.vel - Fl.vel);
-    } else if (MODE == MODE_ACC) {
+        for (int q = 0; q < NVAR; ++q) st_lane(E.acc.p[q], off, F.f[q] - Fl.f[q]);
+        st_lane(E.gp.p[0], off, cG);
+        st_lane(E.gp.p[1], off, cP);
+        st_lane(E.gp.p[2], off, F.vel - Fl.vel);
+    } else if constexpr (MODE == MODE_ACC) {
         // _yextraterm_hllc ("+=", GPUkernels.cu:439-441)
 #pragma unroll
         for (int q = 0; q < NVAR; ++q) {
             const Real t = (in.acc[q] + F.f[q]) - Fl.f[q];
-            if (kFold) st_lane<false>(A.R, q*fs + e, lo, unscaled_stage(A.a) ? A.a*in.R[q] - t : A.a*in.R[q] - dtinvh*t);
-            else       st_lane<false>(acc, q*fs + e, lo, t);
+            if constexpr (kFold) st_lane(E.R.p[q], off, unscaled_stage(A.a) ? A.a*in.R[q] - t : A.a*in.R[q] - dtinvh*t);
+            else       st_lane(E.acc.p[q], off, t);
         }
-        st_lane<false>(acc, A_SUMG*fs + e, lo, in.acc[A_SUMG] + cG);
-        st_lane<false>(acc, A_SUMP*fs + e, lo, in.acc[A_SUMP] + cP);
-        st_lane<false>(acc, A_DIVU*fs + e, lo, in.acc[A_DIVU] + (F.vel - Fl.vel));
+        st_lane(E.gp.p[0], off, in.acc[A_SUMG] + cG);
+        st_lane(E.gp.p[1], off, in.acc[A_SUMP] + cP);
+        st_lane(E.gp.p[2], off, in.acc[A_DIVU] + (F.vel - Fl.vel));
     } else {
         // _zextraterm_hllc + _divergence (+ _update), GPUkernels.cu:812-814,1104-1136,1164-1170
         const Real sG = in.acc[A_SUMG] + cG;
@@ -337,20 +376,20 @@ __device__ __forceinline__ void emit(const StageArgs& A, const Real dtinvh, cons
             // subtraction, so it rounds as the x+y sweep's product would)
             const Real Rx = !kFold ? A.a*in.R[q] : unscaled_stage(A.a) ? __fmul_rn(dtinvh, in.R[q]) : in.R[q];
             const Real Rn = Rx - rhs;
-            if (MODE != MODE_STAGE_NOR) st_lane<false, true>(A.R, q*fs + e, lo, Rn);
-            if (is_stage(MODE)) {
+            if constexpr (MODE != MODE_STAGE_NOR) st_lane<true>(E.R.p[q], off, Rn);
+            if constexpr (is_stage(MODE)) {
                 if (kEPair && q == FE) {
                     // E + b R in binary64, stored as the rounded sum and its
                     // remainder (exact: |remainder| <= half an ulp of the sum)
                     const double Ed = (double(in.u[FE]) + double(in.u[FELO])) + double(A.b) * double(Rn);
                     const Real hi = Real(Ed);
                     un[q] = hi;
-                    st_lane<false, true>(A.uo, q*fs + e, lo, hi);
-                    st_lane<false, true>(A.uo, FELO*fs + e, lo, Real(Ed - double(hi)));
+                    st_lane<true>(E.uo.p[q], off, hi);
+                    st_lane<true>(E.uo.p[FELO], off, Real(Ed - double(hi)));
                     Eun = Ed;
                 } else {
                     un[q] = A.b*Rn + in.u[q];
-                    st_lane<false, true>(A.uo, q*fs + e, lo, un[q]);
+                    st_lane<true>(E.uo.p[q], off, un[q]);
                 }
             }
         }
@@ -382,12 +421,12 @@ struct March
     // std::bool_constant (the peeled steps of an unrolled march)
     template <class FLUX, class EMIT>
     __device__ __forceinline__ void step(const StageArgs& A, const Real dtinvh, const FLUX flux, const EMIT em,
-                                         const LaneIdx& L, const int64_t row_km1, const EmitIn<MODE>& in)
+                                         const EmitPtr<MODE>& E, const uint32_t off_km1, const EmitIn<MODE>& in)
     {
         const CellRec r = reconstruct<Real, kFast>(w0, w1, w2, w3, w4);
         if (flux) {
             const FaceFlux F = riemann<D, Real, kFast>(pm, r.p);
-            if (em) emit<MODE>(A, dtinvh, L, row_km1, in, F, Fl, pGp + pm.G, pPp + pm.P, smax, bad);
+            if (em) emit<MODE>(A, E, dtinvh, off_km1, in, F, Fl, pGp + pm.G, pPp + pm.P, smax, bad);
             Fl = F;
         }
         pm = r.m; pGp = r.p.G; pPp = r.p.P;
@@ -428,22 +467,31 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
     const int s = g.stride(D);
     const int e0 = D == 1 ? g.idx(x, 0, t) : g.idx(x, t, 0);
     // the columns of a wave are consecutive: the first active lane's element is the least
-    const LaneIdx L = lane_idx(e0, e0);
+    const LaneIdx L = lane_idx(e0, e0, (int64_t)c0 * s);
+    constexpr int NEGQ = D == 1 ? FV : FW;   // normal momentum of the marched axis
+    constexpr int FLO = 2 * D;               // its low face
+    const Real* const u0 = A.u + L.base;   // row c0
+    const Bases<NU, const Real> U(u0 - GHOST * (int64_t)s, A.fs);   // row c0 - 3 (y sweep)
+    const EmitPtr<MODE> E(A, L.base);
+    // byte offset of row k (c0 <= k < c1: the launch keeps chunks within 32 bits)
+    auto off = [&](const int k) { return L.lo + (uint32_t)(k - c0) * (uint32_t)s * (uint32_t)sizeof(Real); };
     // the y sweep of a first stage stores its part unscaled and does not read dt
     const Real dtinvh = (MODE == MODE_ACC && unscaled_stage(A.a)) ? Real(0.0f) : stage_dtinvh(A);
     const int64_t fs = A.fs;
+    auto load = [&](const int row, Real* out) {
+        if constexpr (D == 2) return load_row_far(A, u0, L.lo, c0, row, nd, s, FLO, out);
+        else                  return load_row(A, U, L.lo, c0 - GHOST, row, nd, s, FLO, out);
+    };
     constexpr bool kRaw = is_stage(MODE);   // the update needs the raw u of the emitted cell
 
-    constexpr int NEGQ = D == 1 ? FV : FW;   // normal momentum of the marched axis
-    constexpr int FLO = 2 * D;               // its low face
     March<D, MODE> m;
     // raw conserved values of cells k-1 .. k+2 (kept for the register update;
     // the emitted cell k-1 is always interior, so its raw values are exact)
     Real r0[NU], r1[NU], r2[NU], r3[NU], w[NU];
-    r1[NEGQ] *= load_row<false>(A, L, c0 - 2, nd, s, FLO, r1);
-    r2[NEGQ] *= load_row<false>(A, L, c0 - 1, nd, s, FLO, r2);
-    r3[NEGQ] *= load_row<false>(A, L, c0, nd, s, FLO, r3);
-    w[NEGQ] *= load_row<false>(A, L, c0 - 3, nd, s, FLO, w);
+    r1[NEGQ] *= load(c0 - 2, r1);
+    r2[NEGQ] *= load(c0 - 1, r2);
+    r3[NEGQ] *= load(c0, r3);
+    w[NEGQ] *= load(c0 - 3, w);
     m.w1 = prim_of(w);
     m.w2 = prim_of(r1);
     m.w3 = prim_of(r2);
@@ -451,7 +499,7 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
     // software pipeline: raw values of the next incoming cell and the emit
     // operands of the next step are loaded one step ahead
     Real nxt[NU];
-    Real nsg = load_row<false>(A, L, c0 + 1, nd, s, FLO, nxt);
+    Real nsg = load(c0 + 1, nxt);
     EmitIn<MODE> ein, ein_next;
     // one march step at row k.  FLUX: face k-1/2 is solved (k >= c0); EMIT:
     // cell k-1 is written (k >= c0 + 1); PF: row k+3 is prefetched and the
@@ -462,14 +510,14 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
 #pragma unroll
         for (int q = 0; q < NU; ++q) { r0[q] = r1[q]; r1[q] = r2[q]; r2[q] = r3[q]; r3[q] = nxt[q]; }
         const Prim q = prim_of(nxt);  // cell k+2
-        if (PF) nsg = load_row<false>(A, L, k + 3, nd, s, FLO, nxt);
-        if (PF && FLUX) emit_load<MODE>(A, L, (int64_t)k * s, ein_next);   // emitted at step k+1
+        if (PF) nsg = load(k + 3, nxt);
+        if (PF && FLUX) emit_load<MODE>(E, off(k), ein_next);   // emitted at step k+1
         if (kRaw) {
 #pragma unroll
             for (int f = 0; f < NU; ++f) ein.u[f] = r0[f];                   // cell k-1
         }
         m.push(q);
-        m.step(A, dtinvh, FLUX, EMIT, L, (int64_t)(k - 1) * s, ein);
+        m.step(A, dtinvh, FLUX, EMIT, E, off(k - 1), ein);
         ein = ein_next;
     };
     if constexpr (kUnrollMarch) {
@@ -815,9 +863,14 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
     const int e0 = g.idx(xm, 0, z);
     // every lane's element is at least that of the first ghost column of lane
     // 0's plane (lanes left of x = 0 read it on a halo face)
-    const LaneIdx L = lane_idx(e0, g.idx(-GHOST, 0, z));
+    const int r0 = c0 - GHOST;             // the first row of the chunk's stencils
+    const LaneIdx L = lane_idx(e0, g.idx(-GHOST, 0, z), (int64_t)r0 * s);
     const int64_t fs = A.fs;
-    Real* __restrict__ acc = A.acc;
+    // row r0 of the fields; a plane is well under 4 GB, so the rows of a chunk
+    // are within 32-bit offsets
+    const Bases<NU, const Real> U(A.u + L.base, fs);
+    const Bases<NVAR, Real> R((kFold ? A.R : A.acc) + L.base, fs);
+    const Bases<3, Real> gp(A.acc + L.base + A_SUMG * fs, fs);
     // boundary signs of a loaded row: y-momentum by the row's mapping,
     // x-momentum by the lane's (applied where the values are consumed)
     auto fix = [&](Real* o, const Real sgy) {
@@ -827,14 +880,14 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
 
     March<1, MODE_ACC> m;
     Real w[NU];
-    fix(w, load_row<true>(A, L, c0 - 3, g.ny, s, 2, w)); m.w1 = prim_of(w);
-    fix(w, load_row<true>(A, L, c0 - 2, g.ny, s, 2, w)); m.w2 = prim_of(w);
-    fix(w, load_row<true>(A, L, c0 - 1, g.ny, s, 2, w)); m.w3 = prim_of(w);
-    fix(w, load_row<true>(A, L, c0, g.ny, s, 2, w));     m.w4 = prim_of(w);
+    fix(w, load_row(A, U, L.lo, r0, c0 - 3, g.ny, s, 2, w)); m.w1 = prim_of(w);
+    fix(w, load_row(A, U, L.lo, r0, c0 - 2, g.ny, s, 2, w)); m.w2 = prim_of(w);
+    fix(w, load_row(A, U, L.lo, r0, c0 - 1, g.ny, s, 2, w)); m.w3 = prim_of(w);
+    fix(w, load_row(A, U, L.lo, r0, c0, g.ny, s, 2, w));     m.w4 = prim_of(w);
     YRec yrec;
     yrec.start(m.w1, m.w2, m.w3, m.w4);
     Real nxt[NU];
-    Real nsg = load_row<true>(A, L, c0 + 1, g.ny, s, 2, nxt);
+    Real nsg = load_row(A, U, L.lo, r0, c0 + 1, g.ny, s, 2, nxt);
     // a first stage stores its x+y part unscaled and does not read dt
     const bool unscaled = FIRST || unscaled_stage(A.a);
     const Real dtinvh = unscaled ? Real(0.0f) : stage_dtinvh(A);
@@ -844,13 +897,14 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
     auto step = [&](auto FLUX, auto EMIT, auto PF, const int k) {
         fix(nxt, nsg);
         const Prim q = prim_of(nxt);  // row k+2
-        if (PF) nsg = load_row<true>(A, L, k + 3, g.ny, s, 2, nxt);
+        if (PF) nsg = load_row(A, U, L.lo, r0, k + 3, g.ny, s, 2, nxt);
         // folded builds: R of row k-1, emitted below (every lane's address is
         // an interior cell, stored or not)
+        const uint32_t off_km1 = L.lo + (uint32_t)((k - 1 - r0) * s) * (uint32_t)sizeof(Real);
         Real Ro[NVAR];
         if (kFold && EMIT && !FIRST) {
 #pragma unroll
-            for (int f = 0; f < NVAR; ++f) Ro[f] = ld_lane<true>(A.R, L.base + f*fs + (int64_t)(k - 1) * s, L.lo);
+            for (int f = 0; f < NVAR; ++f) Ro[f] = ld_lane(R.p[f], off_km1);
         }
         m.push(q);
         const CellRec ry = yrec.row(m.w0, m.w1, m.w2, m.w3, m.w4);              // row k, y-direction
@@ -866,18 +920,17 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
                 for (int f = 0; f < NVAR; ++f) Fxr.f[f] = from_right(Fxl.f[f]);
                 Fxr.vel = from_right(Fxl.vel);
                 if (store) {
-                    const int64_t e = L.base + (int64_t)(k - 1) * s;   // wave-uniform part
                     const Real cGy = m.pGp + m.pm.G, cPy = m.pPp + m.pm.P;
 #pragma unroll
                     for (int f = 0; f < NVAR; ++f) {
                         const Real t = ((Fxr.f[f] - Fxl.f[f]) + Fy.f[f]) - m.Fl.f[f];
                         // first stage: -t, which is 0 R - t up to the sign of a zero
-                        if (kFold) st_lane<true>(A.R, f*fs + e, L.lo, unscaled ? -t : A.a*Ro[f] - dtinvh*t);
-                        else       st_lane<true>(acc, f*fs + e, L.lo, t);
+                        if (kFold) st_lane(R.p[f], off_km1, unscaled ? -t : A.a*Ro[f] - dtinvh*t);
+                        else       st_lane(R.p[f], off_km1, t);
                     }
-                    st_lane<true, true>(acc, A_SUMG*fs + e, L.lo, (rx.p.G + rx.m.G) + cGy);
-                    st_lane<true, true>(acc, A_SUMP*fs + e, L.lo, (rx.p.P + rx.m.P) + cPy);
-                    st_lane<true, true>(acc, A_DIVU*fs + e, L.lo, (Fxr.vel - Fxl.vel) + (Fy.vel - m.Fl.vel));
+                    st_lane<true>(gp.p[0], off_km1, (rx.p.G + rx.m.G) + cGy);
+                    st_lane<true>(gp.p[1], off_km1, (rx.p.P + rx.m.P) + cPy);
+                    st_lane<true>(gp.p[2], off_km1, (Fxr.vel - Fxl.vel) + (Fy.vel - m.Fl.vel));
                 }
             }
             m.Fl = Fy;
@@ -1628,7 +1681,7 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
         hipLaunchKernelGGL((k_sweep_yz<1, MODE_ACC>), grid, dim3(256), 0, s, g, A, chunk);
     } else {
         const int nb = z_blocks(g);
-        const int chunk = whole ? whole_march(nzr, nb, 2) : pick_chunk(nzr, (int64_t)g.nx * g.ny);
+        const int chunk = std::min(z_march_limit(g), whole ? whole_march(nzr, nb, 2) : pick_chunk(nzr, (int64_t)g.nx * g.ny));
         const dim3 grid(nb, (nzr + chunk - 1) / chunk);
         if (stage == 2)      hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE_NOR>), grid, dim3(256), 0, s, g, A, chunk);
         else if (stage == 1) hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE>), grid, dim3(256), 0, s, g, A, chunk);
