@@ -128,6 +128,12 @@ constexpr int kXCDs = 8;
 // the fused x+y march unrolled by five in the binary32 FAST builds (in the
 // bit-exact and binary64 builds the unrolled march spills)
 constexpr bool kUnrollXY = kFast && !MPCF_F64;
+// the waves of a workgroup of the FAST x+y sweep keep phase (keep_phase)
+// (single-case and batched flat launches: 512^3 step 19.45 -> 18.61 ms, a
+// 24-case ensemble 1.76 -> 1.72 ms; the persistent launches' item loop has
+// barriers of its own that a wave without work reaches early, and does not).
+// The z sweep gains 0.5 % at most and is left alone
+constexpr bool kSyncXY = kFast && !MPCF_F64;
 // likewise the y / z marches (a separate switch: their register budget differs)
 constexpr bool kUnrollMarch = kFast && !MPCF_F64;
 
@@ -755,28 +761,32 @@ __device__ __forceinline__ int xcd_order(const int lin, const int n)
 // FAST: the second difference and its indicator term are formed once per lane
 // and shifted (six shifts and 18 operations up to the indicators, against 4
 // and 25 with shifted first differences)
+template <bool SYNC>
 __device__ __forceinline__ RecT<Real> weno_lanes(const Real c)
 {
     const Real b = from_left(c), d = from_right(c);
     if constexpr (kFast) {
         const Real dbc = c - b, dcd = d - c;
         const Real D = dcd - dbc, Q = weno_term<Real>(D);
-        return weno_fast_core<Real>(b, c, d, dbc, dcd, from_left(D), D, from_right(D), from_left(Q), Q, from_right(Q));
+        const Real Db = from_left(D), Dd = from_right(D), Qb = from_left(Q), Qd = from_right(Q);
+        keep_phase<SYNC>();
+        return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, Qb, Q, Qd);
     } else {
         return weno_cell<Real, kFast>(from_left(b), b, c, d, from_right(d));
     }
 }
+template <bool SYNC>
 __device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c)
 {
     CellRec o;
     RecT<Real> t;
-    t = weno_lanes(c.r); o.m.r = t.m; o.p.r = t.p;
-    t = weno_lanes(c.u); o.m.u = t.m; o.p.u = t.p;
-    t = weno_lanes(c.v); o.m.v = t.m; o.p.v = t.p;
-    t = weno_lanes(c.w); o.m.w = t.m; o.p.w = t.p;
-    t = weno_lanes(c.p); o.m.p = t.m; o.p.p = t.p;
-    t = weno_lanes(c.G); o.m.G = t.m; o.p.G = t.p;
-    t = weno_lanes(c.P); o.m.P = t.m; o.p.P = t.p;
+    t = weno_lanes<SYNC>(c.r); o.m.r = t.m; o.p.r = t.p;
+    t = weno_lanes<SYNC>(c.u); o.m.u = t.m; o.p.u = t.p;
+    t = weno_lanes<SYNC>(c.v); o.m.v = t.m; o.p.v = t.p;
+    t = weno_lanes<SYNC>(c.w); o.m.w = t.m; o.p.w = t.p;
+    t = weno_lanes<SYNC>(c.p); o.m.p = t.m; o.p.p = t.p;
+    t = weno_lanes<SYNC>(c.G); o.m.G = t.m; o.p.G = t.p;
+    t = weno_lanes<SYNC>(c.P); o.m.P = t.m; o.p.P = t.p;
     return o;
 }
 
@@ -786,11 +796,12 @@ struct Diff2 { Real D0, D1, Q0, Q1; };
 
 // y-direction reconstruction of row k of one primitive from rows k-1 .. k+2
 // (b, c, d, e); s holds rows k-1 and k on entry, rows k and k+1 on return
+template <bool SYNC>
 __device__ __forceinline__ Rec weno_march(const Real b, const Real c, const Real d, const Real e, Diff2& s)
 {
     const Real dbc = c - b, dcd = d - c, dde = e - d;
     const Real D2 = dde - dcd, Q2 = weno_term<Real>(D2);
-    const Rec r = weno_fast_core<Real>(b, c, d, dbc, dcd, s.D0, s.D1, D2, s.Q0, s.Q1, Q2);
+    const Rec r = weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, s.D0, s.D1, D2, s.Q0, s.Q1, Q2);
     s.D0 = s.D1; s.D1 = D2;
     s.Q0 = s.Q1; s.Q1 = Q2;
     return r;
@@ -798,6 +809,7 @@ __device__ __forceinline__ Rec weno_march(const Real b, const Real c, const Real
 
 // the y reconstruction of the x+y march: FAST carries the second differences,
 // the other builds evaluate the window as it stands
+template <bool SYNC>
 struct YRec
 {
     Diff2 r, u, v, w, p, G, P;
@@ -822,13 +834,13 @@ struct YRec
         if constexpr (!kFast) return reconstruct<Real, kFast>(A, B, C, D, E);
         CellRec o;
         Rec t;
-        t = weno_march(B.r, C.r, D.r, E.r, r); o.m.r = t.m; o.p.r = t.p;
-        t = weno_march(B.u, C.u, D.u, E.u, u); o.m.u = t.m; o.p.u = t.p;
-        t = weno_march(B.v, C.v, D.v, E.v, v); o.m.v = t.m; o.p.v = t.p;
-        t = weno_march(B.w, C.w, D.w, E.w, w); o.m.w = t.m; o.p.w = t.p;
-        t = weno_march(B.p, C.p, D.p, E.p, p); o.m.p = t.m; o.p.p = t.p;
-        t = weno_march(B.G, C.G, D.G, E.G, G); o.m.G = t.m; o.p.G = t.p;
-        t = weno_march(B.P, C.P, D.P, E.P, P); o.m.P = t.m; o.p.P = t.p;
+        t = weno_march<SYNC>(B.r, C.r, D.r, E.r, r); o.m.r = t.m; o.p.r = t.p;
+        t = weno_march<SYNC>(B.u, C.u, D.u, E.u, u); o.m.u = t.m; o.p.u = t.p;
+        t = weno_march<SYNC>(B.v, C.v, D.v, E.v, v); o.m.v = t.m; o.p.v = t.p;
+        t = weno_march<SYNC>(B.w, C.w, D.w, E.w, w); o.m.w = t.m; o.p.w = t.p;
+        t = weno_march<SYNC>(B.p, C.p, D.p, E.p, p); o.m.p = t.m; o.p.p = t.p;
+        t = weno_march<SYNC>(B.G, C.G, D.G, E.G, G); o.m.G = t.m; o.p.G = t.p;
+        t = weno_march<SYNC>(B.P, C.P, D.P, E.P, P); o.m.P = t.m; o.p.P = t.p;
         return o;
     }
 };
@@ -836,7 +848,9 @@ struct YRec
 // wave `wv` of the x+y sweep over rows [bz * chunk, bz * chunk + chunk).
 // FIRST (folded builds, a = 0 known at launch): R is not read -- the stage
 // multiplies it by zero -- which takes 28 B/cell from that stage's traffic
-template <bool FIRST = false>
+// SYNC: the waves of the workgroup keep phase (keep_phase); all of them run
+// rows of the same chunk, and a wave past the end leaves the kernel
+template <bool FIRST = false, bool SYNC = false>
 __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A, const int chunk,
                                               const int wv, const int bz)
 {
@@ -884,7 +898,7 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
     fix(w, load_row(A, U, L.lo, r0, c0 - 2, g.ny, s, 2, w)); m.w2 = prim_of(w);
     fix(w, load_row(A, U, L.lo, r0, c0 - 1, g.ny, s, 2, w)); m.w3 = prim_of(w);
     fix(w, load_row(A, U, L.lo, r0, c0, g.ny, s, 2, w));     m.w4 = prim_of(w);
-    YRec yrec;
+    YRec<SYNC> yrec;
     yrec.start(m.w1, m.w2, m.w3, m.w4);
     Real nxt[NU];
     Real nsg = load_row(A, U, L.lo, r0, c0 + 1, g.ny, s, 2, nxt);
@@ -909,12 +923,12 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
         m.push(q);
         const CellRec ry = yrec.row(m.w0, m.w1, m.w2, m.w3, m.w4);              // row k, y-direction
         if (FLUX) {
-            const FaceFlux Fy = riemann<1, Real, kFast>(m.pm, ry.p);                // face k-1/2
+            const FaceFlux Fy = riemann<1, Real, kFast, SYNC>(m.pm, ry.p);          // face k-1/2
             if (EMIT) {
                 // x-direction of row k-1 (window slot w1)
-                const CellRec rx = reconstruct_lanes(m.w1);
+                const CellRec rx = reconstruct_lanes<SYNC>(m.w1);
                 const Prim Lm = prim_from_left(rx.m);
-                const FaceFlux Fxl = riemann<0, Real, kFast>(Lm, rx.p);            // face x-1/2
+                const FaceFlux Fxl = riemann<0, Real, kFast, SYNC>(Lm, rx.p);      // face x-1/2
                 FaceFlux Fxr;                                                        // face x+1/2
 #pragma unroll
                 for (int f = 0; f < NVAR; ++f) Fxr.f[f] = from_right(Fxl.f[f]);
@@ -976,7 +990,7 @@ void k_sweep_xy(const Geom g, const StageArgs A, const int chunk)
     __builtin_amdgcn_s_setprio(2);
     const int gx = gridDim.x;
     const int t = xcd_order(blockIdx.x + blockIdx.y * gx, gx * gridDim.y);
-    sweep_xy_body<FIRST>(g, A, chunk, (t % gx) * 4 + threadIdx.y, t / gx);
+    sweep_xy_body<FIRST, kSyncXY>(g, A, chunk, (t % gx) * 4 + threadIdx.y, t / gx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1401,7 +1415,7 @@ void kb_sweep_xy(const BatchDev B, const Real a, const Real b)
     const CaseDesc& C = B.cases[c];
     const int local = blockIdx.x - B.off_xy[c];
     const StageArgs A = case_args(C, B.cur[c], a, b);
-    sweep_xy_body<FIRST>(C.g, A, C.chunk_xy, (local % C.nbx_xy) * 4 + threadIdx.y, local / C.nbx_xy);
+    sweep_xy_body<FIRST, kSyncXY>(C.g, A, C.chunk_xy, (local % C.nbx_xy) * 4 + threadIdx.y, local / C.nbx_xy);
 }
 
 // the z sweep finishes the stage; the last block of each case to finish

@@ -79,6 +79,24 @@ MPCF_HD double mclamp(double x, double lo, double hi) { return fmin(fmax(x, lo),
 template <bool FAST, typename T> MPCF_HD T qdiv(const T a, const T b) { return FAST ? a * mrcp(b) : a / b; }
 template <bool FAST, typename T> MPCF_HD T qsqrt(const T a) { return FAST ? msqrt_fast(a) : msqrt(a); }
 
+// SYNC: the workgroup's waves meet here.  Nothing is exchanged: the barrier
+// keeps waves that march side by side in the same phase of the arithmetic.
+// In the FAST x+y sweep, whose four waves otherwise drift apart at every
+// reciprocal and lane shift, it takes the 512^3 step from 19.45 to 18.61 ms
+// (a scheduling fence alone: 19.56, the barrier without the fence: 19.28).
+// Only for kernels in which every wave of the workgroup runs the same steps.
+template <bool SYNC>
+MPCF_HD void keep_phase()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (SYNC) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#endif
+}
+
 template <typename T>
 struct PrimT { T r, u, v, w, p, G, P; };
 typedef PrimT<Real> Prim;
@@ -149,7 +167,7 @@ template <typename T> MPCF_HD T weno_term(const T D)
 
 // b, c, d: the window's centre three values; dbc = c-b, dcd = d-c; Db, Dc, Dd:
 // the second differences of b, c, d, and Qb, Qc, Qd their terms
-template <typename T>
+template <typename T, bool SYNC = false>
 MPCF_HD RecT<T> weno_fast_core(const T b, const T c, const T d, const T dbc, const T dcd, const T Db, const T Dc,
                                const T Dd, const T Qb, const T Qc, const T Qd)
 {
@@ -161,6 +179,7 @@ MPCF_HD RecT<T> weno_fast_core(const T b, const T c, const T d, const T dbc, con
     const T iB = tB*tB + Qc;
     const T iC = tC*tC + Qd;
     const T rA = mrcp(iA*iA), rB = mrcp(iB*iB), rC = mrcp(iC*iC);
+    keep_phase<SYNC>();
     // The minus state is c + sum_k w_k n_k / 6 with candidates 6 (q_k - c)
     // n0 = 2 tA - (c-b), n1 = (c-b) + 2 (d-c), n2 = 4 (d-c) - (e-d) and
     // weights w ~ (rA, 6 rB, 3 rC).  Written about the central candidate,
@@ -183,8 +202,10 @@ MPCF_HD RecT<T> weno_fast_core(const T b, const T c, const T d, const T dbc, con
     const T qp = CY*k1_3 + 0.5f*AX;
     const T bm = (tB + dcd)*k1_6 + c;              // c + n1/6
     const T bp = c - (tB + dbc)*k1_6;              // c - ((d-c) + 2 (c-b))/6
-    const T om = qm*mrcp(Sm) + bm;
-    const T op = bp - qp*mrcp(Sp);
+    const T iSm = mrcp(Sm), iSp = mrcp(Sp);
+    keep_phase<SYNC>();
+    const T om = qm*iSm + bm;
+    const T op = bp - qp*iSp;
     const T mn = mmin(mmin(b, c), d);
     const T mx = mmax(mmax(b, c), d);
     out.m = mclamp(om, mn, mx);
@@ -289,7 +310,7 @@ template <typename T> struct FaceFluxT { T f[NVAR]; T vel; };
 // 638-662 (y), 934-957 (z).  The states are taken by value: the FAST path
 // selects fields of one side, and selects between loads through references
 // would keep the callers' register-resident march state in memory.
-template <int D, typename T, bool FAST>
+template <int D, typename T, bool FAST, bool SYNC = false>
 MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
 {
     typedef typename Wide<T>::type W;
@@ -310,9 +331,11 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     const T cp2 = qdiv<FAST>(qdiv<FAST>(pp + Pp, Gp) + pp, rp);
     const T cm  = qsqrt<FAST>(cm2);
     const T cp  = qsqrt<FAST>(cp2);
+    keep_phase<SYNC>();
     const T eta_2 = 0.5f*Rr*Rinv*Rinv;
     const T d2    = (cm2 + Rr*cp2)*Rinv + eta_2*(vnp - vnm)*(vnp - vnm);
     const T dd    = qsqrt<FAST>(d2);
+    keep_phase<SYNC>();
     const T ubar  = (vnm + Rr*vnp)*Rinv;
     const T sm = mmin(ubar - dd, vnm - cm);
     const T sp = mmax(ubar + dd, vnp + cp);
@@ -321,6 +344,7 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     const T facm = rm * (sm - vnm);
     const T facp = rp * (sp - vnp);
     const T ss = qdiv<FAST>(pp - pm + vnm*facm - vnp*facp, facm - facp);
+    keep_phase<SYNC>();
 
     FaceFluxT<T> o;
     if constexpr (FAST) {
@@ -336,6 +360,7 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
         const T sk = lt ? sm : sp;
         const T s = lt ? mmin(T(0.0f), sm) : mmax(T(0.0f), sp);
         const T ik = mrcp(sk - ss);
+        keep_phase<SYNC>();
         const T chi = (sk - vn)*ik;
         const T vel = vn + s*(chi - 1.0f);                      // _extraterm_hllc_vel
         const T rv = r*vel;
