@@ -23,6 +23,10 @@ int fail(int code, const std::string& msg);
 // host memcpy of n bytes split over a pool of worker threads (created on first
 // use, kept until the process ends); concurrent callers take turns
 void parallel_copy(void* dst, const void* src, size_t n);
+
+// nh host arrays of `per` bytes each <-> consecutive device memory at dev,
+// ordered on stream s; see mpcf_capi.cpp
+int host_copy(hipStream_t s, void* dev, void* const* host, int nh, size_t per, bool to_device);
 const char* last_error();
 
 }  // namespace detail

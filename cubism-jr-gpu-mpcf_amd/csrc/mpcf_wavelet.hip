@@ -313,11 +313,11 @@ int encode(const float* d_cube, const int n, const float eps, const int half, st
     hipLaunchKernelGGL(k_scatter, grid_for(N3), dim3(256), 0, s, a, n, fl, off, half, vals);
     WL_TRY(hipGetLastError());
     raw.resize(nbits + (size_t)survivors * esz);
-    WL_TRY(hipMemcpyAsync(raw.data(), bits, nbits, hipMemcpyDeviceToHost, s));
-    if (survivors)
-        WL_TRY(hipMemcpyAsync(raw.data() + nbits, vals, (size_t)survivors * esz, hipMemcpyDeviceToHost, s));
-    WL_TRY(hipStreamSynchronize(s));
-    return MPCF_OK;
+    void* dst = raw.data();
+    rc = mpcf::detail::host_copy(s, bits, &dst, 1, nbits, false);
+    if (rc != MPCF_OK || !survivors) return rc;
+    dst = raw.data() + nbits;
+    return mpcf::detail::host_copy(s, vals, &dst, 1, (size_t)survivors * esz, false);
 }
 
 // WaveletCompressorGeneric::decompress into the device cube d_out
@@ -348,10 +348,12 @@ int decode(const unsigned char* raw, const size_t nbytes, const int n, const int
     int* off = (int*)S.get(N3 * 4);
     unsigned char* d_raw = (unsigned char*)S.get(nbytes);
     WL_TRY(S.e);
-    WL_TRY(hipMemcpyAsync(d_raw, raw, nbytes, hipMemcpyHostToDevice, s));
+    void* const src = const_cast<unsigned char*>(raw);
+    int rc = mpcf::detail::host_copy(s, d_raw, &src, 1, nbytes, true);
+    if (rc != MPCF_OK) return rc;
     hipLaunchKernelGGL(k_flags_from_bits, grid_for(N3), dim3(256), 0, s, d_raw, n, fl);
     WL_TRY(hipGetLastError());
-    int rc = exclusive_scan(S, fl, off, N3, s);
+    rc = exclusive_scan(S, fl, off, N3, s);
     if (rc != MPCF_OK) return rc;
     hipLaunchKernelGGL(k_gather, grid_for(N3), dim3(256), 0, s, (const void*)(d_raw + nbits), n, fl, off, half, d_out);
     iwt(d_out, t1, t2, n, s);
@@ -446,9 +448,9 @@ extern "C" int mpcf_wavelet_encode(const float* cube, int n, float threshold, in
     float* d = nullptr;
     WL_TRY(hipMalloc(&d, N3 * 4));
     std::vector<unsigned char> raw;
-    hipError_t e = hipMemcpy(d, cube, N3 * 4, hipMemcpyHostToDevice);
-    int rc = e == hipSuccess ? encode(d, n, threshold, halffloat, raw, nullptr)
-                             : fail(MPCF_EHIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
+    void* const src = const_cast<float*>(cube);
+    int rc = mpcf::detail::host_copy(nullptr, d, &src, 1, (size_t)N3 * 4, true);
+    if (rc == MPCF_OK) rc = encode(d, n, threshold, halffloat, raw, nullptr);
     hipFree(d);
     if (rc != MPCF_OK) return rc;
     *nbytes = (long long)raw.size();
@@ -464,10 +466,8 @@ extern "C" int mpcf_wavelet_decode(const unsigned char* in, long long nbytes, in
     float* d = nullptr;
     WL_TRY(hipMalloc(&d, N3 * 4));
     int rc = decode(in, (size_t)nbytes, n, halffloat, d, nullptr);
-    if (rc == MPCF_OK) {
-        const hipError_t e = hipMemcpy(cube, d, N3 * 4, hipMemcpyDeviceToHost);
-        if (e != hipSuccess) rc = fail(MPCF_EHIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
-    }
+    void* const dst = cube;
+    if (rc == MPCF_OK) rc = mpcf::detail::host_copy(nullptr, d, &dst, 1, (size_t)N3 * 4, false);
     hipFree(d);
     return rc;
 }
