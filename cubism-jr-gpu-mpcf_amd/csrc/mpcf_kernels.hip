@@ -761,8 +761,8 @@ __device__ __forceinline__ int xcd_order(const int lin, const int n)
 // FAST: the second difference and its indicator term are formed once per lane
 // and shifted (six shifts and 18 operations up to the indicators, against 4
 // and 25 with shifted first differences)
-template <bool SYNC>
-__device__ __forceinline__ RecT<Real> weno_lanes(const Real c)
+template <bool SYNC, bool QUICK>
+__device__ __forceinline__ RecT<Real> weno_lanes(const Real c, bool* odd)
 {
     const Real b = from_left(c), d = from_right(c);
     if constexpr (kFast) {
@@ -772,22 +772,36 @@ __device__ __forceinline__ RecT<Real> weno_lanes(const Real c)
         keep_phase<SYNC>();
         return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, Qb, Q, Qd);
     } else {
-        return weno_cell<Real, kFast>(from_left(b), b, c, d, from_right(d));
+        return weno_cell<Real, kFast, QUICK>(from_left(b), b, c, d, from_right(d), odd);
     }
 }
-template <bool SYNC>
-__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c)
+template <bool SYNC, bool QUICK>
+__device__ __forceinline__ CellRec reconstruct_lanes_as(const Prim& c, bool* odd)
 {
     CellRec o;
     RecT<Real> t;
-    t = weno_lanes<SYNC>(c.r); o.m.r = t.m; o.p.r = t.p;
-    t = weno_lanes<SYNC>(c.u); o.m.u = t.m; o.p.u = t.p;
-    t = weno_lanes<SYNC>(c.v); o.m.v = t.m; o.p.v = t.p;
-    t = weno_lanes<SYNC>(c.w); o.m.w = t.m; o.p.w = t.p;
-    t = weno_lanes<SYNC>(c.p); o.m.p = t.m; o.p.p = t.p;
-    t = weno_lanes<SYNC>(c.G); o.m.G = t.m; o.p.G = t.p;
-    t = weno_lanes<SYNC>(c.P); o.m.P = t.m; o.p.P = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.r, odd); o.m.r = t.m; o.p.r = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.u, odd); o.m.u = t.m; o.p.u = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.v, odd); o.m.v = t.m; o.p.v = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.w, odd); o.m.w = t.m; o.p.w = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.p, odd); o.m.p = t.m; o.p.p = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.G, odd); o.m.G = t.m; o.p.G = t.p;
+    t = weno_lanes<SYNC, QUICK>(c.P, odd); o.m.P = t.m; o.p.P = t.p;
     return o;
+}
+// as reconstruct(): the bit-exact builds take the quick quotients, and the
+// IEEE ones where a lane's window needs them
+template <bool SYNC>
+__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c)
+{
+    if constexpr (!kFast) {
+        bool odd = false;
+        CellRec o = reconstruct_lanes_as<SYNC, true>(c, &odd);
+        if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_lanes_as<SYNC, false>(c, nullptr);
+        return o;
+    } else {
+        return reconstruct_lanes_as<SYNC, false>(c, nullptr);
+    }
 }
 
 // what a FAST march along y carries of one primitive besides the window: the
@@ -1327,7 +1341,10 @@ __global__ void k_test_weno(const int n, const Real* __restrict__ in5, Real* __r
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const Real* a = in5 + 5*(int64_t)i;
-    const Rec r = weno_cell<Real, kFast>(a[0], a[1], a[2], a[3], a[4]);
+    // as the sweeps do: quick quotients, and the IEEE ones where a lane's window needs them
+    bool odd = false;
+    Rec r = weno_cell<Real, kFast, !kFast>(a[0], a[1], a[2], a[3], a[4], &odd);
+    if (any_lane(odd)) r = weno_cell<Real, kFast>(a[0], a[1], a[2], a[3], a[4]);
     m[i] = r.m; p[i] = r.p;
 }
 

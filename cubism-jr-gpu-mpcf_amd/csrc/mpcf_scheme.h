@@ -28,6 +28,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cmath>
+#include <type_traits>
 #include "mpcf_geom.h"
 
 namespace mpcf {
@@ -40,6 +41,34 @@ template <typename T> struct Wide { typedef double type; };
 MPCF_HD float mmin(float a, float b) { return fminf(a, b); }
 MPCF_HD float mmax(float a, float b) { return fmaxf(a, b); }
 MPCF_HD float msqrt(float a) { return sqrtf(a); }
+MPCF_HD float mabs(float a) { return fabsf(a); }
+// the least / greatest of three, as fminf / fmaxf of them in turn: one
+// instruction, without the ones that quiet signalling NaNs of loaded or
+// lane-shifted operands first
+MPCF_HD float mmin3(float a, float b, float c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return fminf(fminf(a, b), c);
+#endif
+}
+MPCF_HD float mmax3(float a, float b, float c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return fmaxf(fmaxf(a, b), c);
+#endif
+}
+MPCF_HD double mmin3(double a, double b, double c) { return fmin(fmin(a, b), c); }
+MPCF_HD double mmax3(double a, double b, double c) { return fmax(fmax(a, b), c); }
+template <typename T> MPCF_HD T mmin3(const T a, const T b, const T c) { return mmin(mmin(a, b), c); }
+template <typename T> MPCF_HD T mmax3(const T a, const T b, const T c) { return mmax(mmax(a, b), c); }
 MPCF_HD double mmin(double a, double b) { return fmin(a, b); }
 MPCF_HD double mmax(double a, double b) { return fmax(a, b); }
 MPCF_HD double msqrt(double a) { return sqrt(a); }
@@ -64,7 +93,7 @@ MPCF_HD float msqrt_fast(float a)
 #endif
 }
 
-// x clamped to [lo, hi] for lo <= hi: one v_med3_f32 on the device (FAST)
+// x clamped to [lo, hi] for lo <= hi: one v_med3_f32 on the device
 MPCF_HD float mclamp(float x, float lo, float hi)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -78,6 +107,64 @@ MPCF_HD double mclamp(double x, double lo, double hi) { return fmin(fmax(x, lo),
 // a / b: IEEE division (bit-exact build) or a * rcp(b) (FAST)
 template <bool FAST, typename T> MPCF_HD T qdiv(const T a, const T b) { return FAST ? a * mrcp(b) : a / b; }
 template <bool FAST, typename T> MPCF_HD T qsqrt(const T a) { return FAST ? msqrt_fast(a) : msqrt(a); }
+
+// Correctly rounded reciprocal, quotient and square root for operands in a
+// safe exponent range: the compiler's IEEE sequences without the steps that
+// scale and repair extreme operands (f32 quotient 6 instructions, not 11, of
+// which 4 run at half rate; square root 5, not 14; f64 reciprocal 6, not 11).
+// The callers check the range and fall back to the IEEE operation.
+//  * rcp_rn(float): one Newton step from v_rcp_f32 gives the correctly rounded
+//    reciprocal of each of the 2^23 significands (all of them tried on the
+//    device).
+//  * div_rn: with a correctly rounded reciprocal one residual correction of
+//    a*y rounds correctly.  The error before the last rounding is below 2.25
+//    2^-24 units in the last place, so only quotients that close to a rounding
+//    midpoint could fail; these are the 2.7e8 significand pairs with
+//    |2^24 a - m b| or |2^25 a - m b| <= 24, all of which were tried.
+//  * sqrt_rn: all 2^24 significands and exponent parities were tried.
+//  * rcp_rn(double): a cubic step from v_rcp_f64 (2^-24.3) is within one unit
+//    in the last place, and Markstein's last step y + y (1 - b y) then rounds
+//    correctly (unless b's significand is all ones, which 10 i^2 of a binary32
+//    i never is; 4.3e9 random b and the 65536 significands below all ones
+//    were tried).
+#if defined(__HIP_DEVICE_COMPILE__)
+template <typename T> constexpr bool kQuick = std::is_floating_point<T>::value;
+MPCF_HD float rcp_rn(const float b)
+{
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+MPCF_HD double rcp_rn(const double b)
+{
+    const double y0 = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, y0, 1.0);
+    const double y = __builtin_fma(y0, __builtin_fma(e, e, e), y0);
+    return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+}
+// a / b with y = rcp_rn(b)
+MPCF_HD float div_rn(const float a, const float b, const float y)
+{
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+MPCF_HD float sqrt_rn(const float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+}
+// zero, subnormal, infinite or NaN
+MPCF_HD bool not_normal(const float x) { return __builtin_amdgcn_classf(x, 0x2f7); }
+MPCF_HD bool not_normal(const double x) { return __builtin_amdgcn_class(x, 0x2f7); }
+MPCF_HD bool any_lane(const bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; }
+#else
+template <typename T> constexpr bool kQuick = false;
+template <typename T> MPCF_HD T rcp_rn(const T b) { return T(1.0) / b; }
+template <typename T> MPCF_HD T div_rn(const T a, const T b, const T) { return a / b; }
+template <typename T> MPCF_HD T sqrt_rn(const T x) { return msqrt(x); }
+template <typename T> MPCF_HD bool not_normal(const T) { return false; }
+MPCF_HD bool any_lane(const bool b) { return b; }
+#endif
 
 // SYNC: the workgroup's waves meet here.  Nothing is exchanged: the barrier
 // keeps waves that march side by side in the same phase of the arithmetic.
@@ -221,8 +308,13 @@ MPCF_HD RecT<T> weno_fast_diff(const T b, const T c, const T d, const T dab, con
     return weno_fast_core<T>(b, c, d, dbc, dcd, Db, Dc, Dd, weno_term(Db), weno_term(Dc), weno_term(Dd));
 }
 
-template <typename T, bool FAST>
-MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e)
+// QUICK (bit-exact builds on the device): the five reciprocals by rcp_rn, which
+// rounds like the division for the indicators of any sane window; `odd` is set
+// where the product of the indicators (binary32) or of their scaled squares
+// (binary64) is not a normal number, and the caller then evaluates the window
+// again without QUICK
+template <typename T, bool FAST, bool QUICK = false>
+MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e, bool* odd = nullptr)
 {
     typedef typename Wide<T>::type W;
     const T k4_3 = T(4./3.), k19_3 = T(19./3.), k11_3 = T(11./3.);
@@ -254,30 +346,40 @@ MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e)
         const T k1_3 = T(1./3.), k7_6 = T(7./6.), k11_6 = T(11./6.);
         const T k1_6 = T(1./6.), k5_6 = T(5./6.), mk1_6 = T(-(1./6.));
         // binary64: the reference writes the literal 10.0 (GPUonly.cuh:111-113,150-152)
-        const W rA = W(1.0) / (10.0*W(iA)*W(iA));
-        const W rB = W(1.0) / (10.0*W(iB)*W(iB));
-        const W rC = W(1.0) / (10.0*W(iC)*W(iC));
+        const W xA = 10.0*W(iA)*W(iA), xB = 10.0*W(iB)*W(iB), xC = 10.0*W(iC)*W(iC);
+        W rA, rB, rC;
+        if constexpr (QUICK) {
+            if constexpr (sizeof(T) == 4) *odd = *odd || not_normal(iA*iB*iC);
+            else                          *odd = *odd || not_normal(xA*xB*xC);
+            rA = rcp_rn(xA); rB = rcp_rn(xB); rC = rcp_rn(xC);
+        } else {
+            rA = W(1.0) / xA; rB = W(1.0) / xB; rC = W(1.0) / xC;
+        }
         const T mA0 = T(rA), mA1 = T(6.0*rB), mA2 = T(3.0*rC);
         const T pA0 = T(rC), pA1 = mA1,       pA2 = T(3.0*rA);
         {   // _weno_minus(a,b,c,d,e)
             const T sum = mA0 + mA1 + mA2;
-            const T inv = qdiv<FAST>(T(1.0f), sum);
+            T inv;
+            if constexpr (QUICK) inv = rcp_rn(sum);
+            else                 inv = qdiv<FAST>(T(1.0f), sum);
             const T w0 = mA0 * inv, w1 = mA1 * inv;
             const T w2 = T(1.0f) - w0 - w1;
             out.m = w0*(k1_3*a - k7_6*b + k11_6*c) + w1*(mk1_6*b + k5_6*c + k1_3*d) + w2*(k1_3*c + k5_6*d - k1_6*e);
         }
         {   // _weno_pluss(a,b,c,d,e)  (its b..f are this cell's a..e)
             const T sum = pA0 + pA1 + pA2;
-            const T inv = qdiv<FAST>(T(1.0f), sum);
+            T inv;
+            if constexpr (QUICK) inv = rcp_rn(sum);
+            else                 inv = qdiv<FAST>(T(1.0f), sum);
             const T w0 = pA0 * inv, w1 = pA1 * inv;
             const T w2 = T(1.0f) - w0 - w1;
             out.p = w0*(k1_3*e - k7_6*d + k11_6*c) + w1*(mk1_6*d + k5_6*c + k1_3*b) + w2*(k1_3*c + k5_6*b - k1_6*a);
         }
         // clipping to the three central cells (identical bounds for both states)
-        const T mn = mmin(mmin(b, c), d);
-        const T mx = mmax(mmax(b, c), d);
-        out.m = mmin(mmax(out.m, mn), mx);
-        out.p = mmin(mmax(out.p, mn), mx);
+        const T mn = mmin3(b, c, d);
+        const T mx = mmax3(b, c, d);
+        out.m = mclamp(out.m, mn, mx);   // NaN: the lower bound, as the minimum of the maximum
+        out.p = mclamp(out.p, mn, mx);
         return out;
     }
 }
@@ -285,20 +387,34 @@ MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e)
 // one cell's reconstructed face states in one direction
 template <typename T> struct CellRecT { PrimT<T> m, p; };
 
+template <typename T, bool FAST, bool QUICK>
+MPCF_HD CellRecT<T> reconstruct_as(const PrimT<T>& A, const PrimT<T>& B, const PrimT<T>& C, const PrimT<T>& D,
+                                   const PrimT<T>& E, bool* odd)
+{
+    CellRecT<T> o;
+    RecT<T> t;
+    t = weno_cell<T, FAST, QUICK>(A.r, B.r, C.r, D.r, E.r, odd); o.m.r = t.m; o.p.r = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.u, B.u, C.u, D.u, E.u, odd); o.m.u = t.m; o.p.u = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.v, B.v, C.v, D.v, E.v, odd); o.m.v = t.m; o.p.v = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.w, B.w, C.w, D.w, E.w, odd); o.m.w = t.m; o.p.w = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.p, B.p, C.p, D.p, E.p, odd); o.m.p = t.m; o.p.p = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.G, B.G, C.G, D.G, E.G, odd); o.m.G = t.m; o.p.G = t.p;
+    t = weno_cell<T, FAST, QUICK>(A.P, B.P, C.P, D.P, E.P, odd); o.m.P = t.m; o.p.P = t.p;
+    return o;
+}
+
 template <typename T, bool FAST>
 MPCF_HD CellRecT<T> reconstruct(const PrimT<T>& A, const PrimT<T>& B, const PrimT<T>& C, const PrimT<T>& D,
                                 const PrimT<T>& E)
 {
-    CellRecT<T> o;
-    RecT<T> t;
-    t = weno_cell<T, FAST>(A.r, B.r, C.r, D.r, E.r); o.m.r = t.m; o.p.r = t.p;
-    t = weno_cell<T, FAST>(A.u, B.u, C.u, D.u, E.u); o.m.u = t.m; o.p.u = t.p;
-    t = weno_cell<T, FAST>(A.v, B.v, C.v, D.v, E.v); o.m.v = t.m; o.p.v = t.p;
-    t = weno_cell<T, FAST>(A.w, B.w, C.w, D.w, E.w); o.m.w = t.m; o.p.w = t.p;
-    t = weno_cell<T, FAST>(A.p, B.p, C.p, D.p, E.p); o.m.p = t.m; o.p.p = t.p;
-    t = weno_cell<T, FAST>(A.G, B.G, C.G, D.G, E.G); o.m.G = t.m; o.p.G = t.p;
-    t = weno_cell<T, FAST>(A.P, B.P, C.P, D.P, E.P); o.m.P = t.m; o.p.P = t.p;
-    return o;
+    if constexpr (!FAST && kQuick<T>) {
+        bool odd = false;
+        CellRecT<T> o = reconstruct_as<T, FAST, true>(A, B, C, D, E, &odd);
+        if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_as<T, FAST, false>(A, B, C, D, E, nullptr);
+        return o;
+    } else {
+        return reconstruct_as<T, FAST, false>(A, B, C, D, E, nullptr);
+    }
 }
 
 // fluxes at one face, in field order, plus the HLLC face velocity of the
@@ -310,8 +426,12 @@ template <typename T> struct FaceFluxT { T f[NVAR]; T vel; };
 // 638-662 (y), 934-957 (z).  The states are taken by value: the FAST path
 // selects fields of one side, and selects between loads through references
 // would keep the callers' register-resident march state in memory.
-template <int D, typename T, bool FAST, bool SYNC = false>
-MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
+// QUICK (bit-exact binary32 build on the device): quotients and square roots by
+// div_rn and sqrt_rn, except the star speed, whose numerator fades through
+// every magnitude ahead of a wave; `odd` is set where an operand or result is
+// outside [2^-40, 2^40], and riemann then solves the face again without QUICK.
+template <int D, typename T, bool FAST, bool SYNC, bool QUICK>
+MPCF_HD FaceFluxT<T> riemann_as(const PrimT<T> L, const PrimT<T> Rt, bool* odd)
 {
     typedef typename Wide<T>::type W;
     // normal and the two transverse velocities in the order _hllc_e receives them
@@ -325,16 +445,29 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     const T Gm = L.G, Gp = Rt.G, Pm = L.P, Pp = Rt.P;
 
     // _char_vel_einfeldt (GPUonly.cuh:823-846)
-    const T Rr   = qsqrt<FAST>(qdiv<FAST>(rp, rm));
-    const T Rinv = qdiv<FAST>(T(1.0f), 1.0f + Rr);
-    const T cm2 = qdiv<FAST>(qdiv<FAST>(pm + Pm, Gm) + pm, rm);
-    const T cp2 = qdiv<FAST>(qdiv<FAST>(pp + Pp, Gp) + pp, rp);
-    const T cm  = qsqrt<FAST>(cm2);
-    const T cp  = qsqrt<FAST>(cp2);
+    T Rr, Rinv, cm2, cp2, cm, cp;
+    if constexpr (QUICK) {
+        const T im = rcp_rn(rm);
+        Rr   = sqrt_rn(div_rn(rp, rm, im));
+        Rinv = rcp_rn(1.0f + Rr);
+        cm2  = div_rn(div_rn(pm + Pm, Gm, rcp_rn(Gm)) + pm, rm, im);
+        cp2  = div_rn(div_rn(pp + Pp, Gp, rcp_rn(Gp)) + pp, rp, rcp_rn(rp));
+        cm   = sqrt_rn(cm2);
+        cp   = sqrt_rn(cp2);
+    } else {
+        Rr   = qsqrt<FAST>(qdiv<FAST>(rp, rm));
+        Rinv = qdiv<FAST>(T(1.0f), 1.0f + Rr);
+        cm2 = qdiv<FAST>(qdiv<FAST>(pm + Pm, Gm) + pm, rm);
+        cp2 = qdiv<FAST>(qdiv<FAST>(pp + Pp, Gp) + pp, rp);
+        cm  = qsqrt<FAST>(cm2);
+        cp  = qsqrt<FAST>(cp2);
+    }
     keep_phase<SYNC>();
     const T eta_2 = 0.5f*Rr*Rinv*Rinv;
     const T d2    = (cm2 + Rr*cp2)*Rinv + eta_2*(vnp - vnm)*(vnp - vnm);
-    const T dd    = qsqrt<FAST>(d2);
+    T dd;
+    if constexpr (QUICK) dd = sqrt_rn(d2);
+    else                 dd = qsqrt<FAST>(d2);
     keep_phase<SYNC>();
     const T ubar  = (vnm + Rr*vnp)*Rinv;
     const T sm = mmin(ubar - dd, vnm - cm);
@@ -386,8 +519,24 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     const int sign_star = ss == 0.0f ? 0 : (ss < 0.0f ? -1 : 1);
     const T s_minus = mmin(T(0.0f), sm);
     const T s_pluss = mmax(T(0.0f), sp);
-    const T chi_m = qdiv<FAST>(sm - vnm, sm - ss);
-    const T chi_p = qdiv<FAST>(sp - vnp, sp - ss);
+    const T am = sm - vnm, ap = sp - vnp, bm = sm - ss, bp = sp - ss;
+    T chi_m, chi_p, pam, pap;                                    // pam = pm / (sm - vnm)
+    if constexpr (QUICK) {
+        chi_m = div_rn(am, bm, rcp_rn(bm));
+        chi_p = div_rn(ap, bp, rcp_rn(bp));
+        pam = div_rn(pm, am, rcp_rn(am));
+        pap = div_rn(pp, ap, rcp_rn(ap));
+        const T lo = mmin3(mmin3(mmin3(rm, rp, Gm), mmin3(Gp, pm + Pm, pp + Pp), mmin3(cm2, cp2, d2)),
+                           mmin3(mabs(am), mabs(ap), mabs(bm)), mmin3(mabs(bp), mabs(pm), mabs(pp)));
+        const T hi = mmax3(mmax3(mmax3(rm, rp, Gm), mmax3(Gp, pm + Pm, pp + Pp), mmax3(cm2, cp2, d2)),
+                           mmax3(mabs(am), mabs(ap), mabs(bm)), mmax3(mabs(bp), mabs(pm), mabs(pp)));
+        *odd = !(lo >= T(0x1p-40f) && hi <= T(0x1p40f));
+    } else {
+        chi_m = qdiv<FAST>(am, bm);
+        chi_p = qdiv<FAST>(ap, bp);
+        pam = qdiv<FAST>(pm, am);
+        pap = qdiv<FAST>(pp, ap);
+    }
     const float wl = 0.5f*(1 + sign_star);
     const float wr = 0.5f*(1 - sign_star);
     const double wr_d = 0.5*(1 - sign_star);
@@ -427,8 +576,8 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     {
         const T qm = Gm*pm + Pm + 0.5f*rm*(vnm*vnm + v1m*v1m + v2m*v2m);
         const T qp = Gp*pp + Pp + 0.5f*rp*(vnp*vnp + v1p*v1p + v2p*v2p);
-        const T q_deltam = chi_m*(qm + (ss - vnm)*(rm*ss + qdiv<FAST>(pm, sm - vnm))) - qm;
-        const T q_deltap = chi_p*(qp + (ss - vnp)*(rp*ss + qdiv<FAST>(pp, sp - vnp))) - qp;
+        const T q_deltam = chi_m*(qm + (ss - vnm)*(rm*ss + pam)) - qm;
+        const T q_deltap = chi_p*(qp + (ss - vnp)*(rp*ss + pap)) - qp;
         const T fm = vnm*(qm + pm);
         const T fp = vnp*(qp + pp);
         fe = wl * (fm + s_minus*q_deltam) + wr * (fp + s_pluss*q_deltap);
@@ -447,6 +596,19 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
         o.vel = wl*(vnm + s_minus*chim1) + wr*(vnp + s_pluss*chip1);
     }
     return o;
+}
+
+template <int D, typename T, bool FAST, bool SYNC = false>
+MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
+{
+    if constexpr (!FAST && kQuick<T> && sizeof(T) == 4) {
+        bool odd = false;
+        FaceFluxT<T> o = riemann_as<D, T, FAST, SYNC, true>(L, Rt, &odd);
+        if (__builtin_expect(any_lane(odd), 0)) o = riemann_as<D, T, FAST, SYNC, false>(L, Rt, nullptr);
+        return o;
+    } else {
+        return riemann_as<D, T, FAST, SYNC, false>(L, Rt, nullptr);
+    }
 }
 
 } // namespace mpcf
