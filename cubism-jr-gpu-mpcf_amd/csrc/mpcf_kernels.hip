@@ -758,19 +758,18 @@ __device__ __forceinline__ int xcd_order(const int lin, const int n)
 }
 
 // x-direction reconstruction of each lane's cell from its lane neighbours.
-// FAST: the second difference and its indicator term are formed once per lane
-// and shifted (six shifts and 18 operations up to the indicators, against 4
-// and 25 with shifted first differences)
+// FAST: the second difference is formed once per lane and shifted (a lane's Db
+// is its left neighbour's Dc, the same subtractions of the same values)
 template <bool SYNC, bool QUICK>
 __device__ __forceinline__ RecT<Real> weno_lanes(const Real c, bool* odd)
 {
     const Real b = from_left(c), d = from_right(c);
     if constexpr (kFast) {
         const Real dbc = c - b, dcd = d - c;
-        const Real D = dcd - dbc, Q = weno_term<Real>(D);
-        const Real Db = from_left(D), Dd = from_right(D), Qb = from_left(Q), Qd = from_right(Q);
+        const Real D = dcd - dbc;
+        const Real Db = from_left(D), Dd = from_right(D);
         keep_phase<SYNC>();
-        return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, Qb, Q, Qd);
+        return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, weno_kD<Real>(Db), weno_kD<Real>(D), weno_kD<Real>(Dd));
     } else {
         return weno_cell<Real, kFast, QUICK>(from_left(b), b, c, d, from_right(d), odd);
     }
@@ -805,8 +804,8 @@ __device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c)
 }
 
 // what a FAST march along y carries of one primitive besides the window: the
-// second differences of the two cells before the newest and their terms
-struct Diff2 { Real D0, D1, Q0, Q1; };
+// second differences of the two cells before the newest and their products
+struct Diff2 { Real D0, D1, k0, k1; };
 
 // y-direction reconstruction of row k of one primitive from rows k-1 .. k+2
 // (b, c, d, e); s holds rows k-1 and k on entry, rows k and k+1 on return
@@ -814,10 +813,10 @@ template <bool SYNC>
 __device__ __forceinline__ Rec weno_march(const Real b, const Real c, const Real d, const Real e, Diff2& s)
 {
     const Real dbc = c - b, dcd = d - c, dde = e - d;
-    const Real D2 = dde - dcd, Q2 = weno_term<Real>(D2);
-    const Rec r = weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, s.D0, s.D1, D2, s.Q0, s.Q1, Q2);
+    const Real D2 = dde - dcd, k2 = weno_kD<Real>(D2);
+    const Rec r = weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, s.D0, s.D1, D2, s.k0, s.k1, k2);
     s.D0 = s.D1; s.D1 = D2;
-    s.Q0 = s.Q1; s.Q1 = Q2;
+    s.k0 = s.k1; s.k1 = k2;
     return r;
 }
 
@@ -832,8 +831,8 @@ struct YRec
     static __device__ __forceinline__ Diff2 first(const Real a, const Real b, const Real c, const Real d)
     {
         Diff2 s;
-        s.D0 = (c - b) - (b - a); s.Q0 = weno_term<Real>(s.D0);
-        s.D1 = (d - c) - (c - b); s.Q1 = weno_term<Real>(s.D1);
+        s.D0 = (c - b) - (b - a); s.k0 = weno_kD<Real>(s.D0);
+        s.D1 = (d - c) - (c - b); s.k1 = weno_kD<Real>(s.D1);
         return s;
     }
     __device__ __forceinline__ void start(const Prim& a, const Prim& b, const Prim& c, const Prim& d)

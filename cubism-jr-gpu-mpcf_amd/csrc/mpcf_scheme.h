@@ -237,34 +237,30 @@ MPCF_HD PrimT<T> to_prim(T r, T ru, T rv, T rw, T E, T G, T P, T Elo = T())
 // (GPUonly.cuh:99-194; WENOEPS = 1e-6, Makefile.config:15)
 template <typename T> struct RecT { T m, p; };
 
-// The FAST reconstruction works on the second differences of the window and
-// one term of the smoothness indicators that depends on them alone.  Cell j's
-// second difference D_j = (j+1 - j) - (j - j-1) and term Q_j serve the windows
-// of cells j-1, j and j+1, so a caller forms them once per cell and hands them
-// on: from row to row of a march, or from lane to lane.
-// Q: the indicators times 4 are 13/3 D^2 + t^2 + 4 eps, each exactly 4 times
-// 13/12 D^2 + 1/4 t^2 + eps (a power-of-two scale of every operand) with one
-// product fewer; the normalised weights depend only on their ratios.
-template <typename T> MPCF_HD T weno_term(const T D)
-{
-    const T k13_3 = 4.0f*T(13./12.);
-    const T eps4 = 4.0f*T(1e-6);
-    return D*(k13_3*D) + eps4;
-}
+// The FAST reconstruction works on the second differences of the window, D_j =
+// (j+1 - j) - (j - j-1) at cell j, and their products k D_j with the indicators'
+// coefficient.  Both serve the windows of cells j-1, j and j+1, so a caller
+// forms them once per cell and hands them on: from row to row of a march, or
+// from lane to lane.
+template <typename T> MPCF_HD T weno_kD(const T D) { return (4.0f*T(13./12.))*D; }
 
 // b, c, d: the window's centre three values; dbc = c-b, dcd = d-c; Db, Dc, Dd:
-// the second differences of b, c, d, and Qb, Qc, Qd their terms
+// the second differences of b, c, d, and kb, kc, kd = weno_kD of them
 template <typename T, bool SYNC = false>
 MPCF_HD RecT<T> weno_fast_core(const T b, const T c, const T d, const T dbc, const T dcd, const T Db, const T Dc,
-                               const T Dd, const T Qb, const T Qc, const T Qd)
+                               const T Dd, const T kb, const T kc, const T kd)
 {
     RecT<T> out;
     const T tA = Db + 2.0f*dbc;                               // a - 4b + 3c
     const T tB = dbc + dcd;                                   // d - b
     const T tC = Dd - 2.0f*dcd;                               // 3c - 4d + e
-    const T iA = tA*tA + Qb;
-    const T iB = tB*tB + Qc;
-    const T iC = tC*tC + Qd;
+    // the indicators times 4, 13/3 D^2 + t^2 + 4 eps: each is exactly 4 times
+    // 13/12 D^2 + 1/4 t^2 + eps (a power-of-two scale of every operand), with
+    // one product fewer; the normalised weights depend only on their ratios
+    const T eps4 = 4.0f*T(1e-6);
+    const T iA = Db*kb + (tA*tA + eps4);
+    const T iB = Dc*kc + (tB*tB + eps4);
+    const T iC = Dd*kd + (tC*tC + eps4);
     const T rA = mrcp(iA*iA), rB = mrcp(iB*iB), rC = mrcp(iC*iC);
     keep_phase<SYNC>();
     // The minus state is c + sum_k w_k n_k / 6 with candidates 6 (q_k - c)
@@ -305,7 +301,7 @@ template <typename T>
 MPCF_HD RecT<T> weno_fast_diff(const T b, const T c, const T d, const T dab, const T dbc, const T dcd, const T dde)
 {
     const T Db = dbc - dab, Dc = dcd - dbc, Dd = dde - dcd;
-    return weno_fast_core<T>(b, c, d, dbc, dcd, Db, Dc, Dd, weno_term(Db), weno_term(Dc), weno_term(Dd));
+    return weno_fast_core<T>(b, c, d, dbc, dcd, Db, Dc, Dd, weno_kD(Db), weno_kD(Dc), weno_kD(Dd));
 }
 
 // QUICK (bit-exact builds on the device): the five reciprocals by rcp_rn, which
@@ -492,17 +488,14 @@ MPCF_HD FaceFluxT<T> riemann_as(const PrimT<T> L, const PrimT<T> Rt, bool* odd)
         const T v1 = lt ? v1m : v1p, v2 = lt ? v2m : v2p;
         const T sk = lt ? sm : sp;
         const T s = lt ? mmin(T(0.0f), sm) : mmax(T(0.0f), sp);
-        const T ik = mrcp(sk - ss);
+        const T chi = qdiv<FAST>(sk - vn, sk - ss);
         keep_phase<SYNC>();
-        const T chi = (sk - vn)*ik;
         const T vel = vn + s*(chi - 1.0f);                      // _extraterm_hllc_vel
         const T rv = r*vel;
         const T rvn = r*vn;
         const T fpv = rvn*vn + p + s*(r*ss*chi - rvn);          // _hllc_pvel
         const T E = G*p + P + 0.5f*r*(vn*vn + v1*v1 + v2*v2);   // _hllc_e
-        // chi / (sk - vn) = 1 / (sk - ss): the pressure term needs no quotient of its own
-        const T dv = ss - vn;
-        const T fe = vn*(E + p) + s*(chi*(E + dv*(r*ss)) + dv*(p*ik) - E);
+        const T fe = vn*(E + p) + s*(chi*(E + (ss - vn)*(r*ss + qdiv<FAST>(p, sk - vn))) - E);
         o.f[FR] = rv;
         if (D == 0) { o.f[FU] = fpv;    o.f[FV] = rv*v1; o.f[FW] = rv*v2; }
         if (D == 1) { o.f[FU] = rv*v1;  o.f[FV] = fpv;   o.f[FW] = rv*v2; }
