@@ -61,6 +61,17 @@ inline Geom make_geom(int nx, int ny, int nz)
     return g;
 }
 
+// workgroups of the speed-of-sound reduction: four waves each, four rows a wave
+// at a time.  Each block ends with two atomics on one cache line, which take
+// turns, so there are no more blocks than keep the memory busy: two million
+// cells 22 us with at most 512 blocks, 43 with 2048 and one row at a time (and
+// 59 with a device-scope fence per block); 512^3 632, 656 and 715 us
+inline int sos_blocks(const Geom& g)
+{
+    const int nb = (g.ny * g.nz + 15) / 16;
+    return nb < 512 ? nb : 512;
+}
+
 // the longest z march: the z sweep addresses the rows of a chunk by 32-bit byte
 // offsets from its first row (binary64 storage, less two planes for the lanes)
 inline int z_march_limit(const Geom& g)

@@ -239,8 +239,7 @@ inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const 
     parity::z_grid(c->g, d.chunk_z, dims);
     d.nbx_z = dims[0]; d.nby_z = dims[1];
     blocks[1] = dims[0] * dims[1] * dims[2];
-    const int rows4 = (c->g.ny * c->g.nz + 3) / 4;
-    d.nb_sos = rows4 < 2048 ? rows4 : 2048;
+    d.nb_sos = sos_blocks(c->g);
     blocks[2] = d.nb_sos;
     (void)cur;
 }

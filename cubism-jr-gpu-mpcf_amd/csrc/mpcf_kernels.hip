@@ -92,13 +92,22 @@ __device__ __forceinline__ SosT sos_cell(const bool cpu_form, const SosT r, cons
     return s;
 }
 
-// moves the maximum (and flag) folded into the previous step's last stage to
-// the reduction targets, where sos_finalize reads them
-__device__ __forceinline__ void take_folded(StepState* st)
+// a maximum speed of sound and its flag as a reduction or a step's last stage
+// left them
+struct SosIn { SosT sos; unsigned bad; };
+
+// the maximum and flag folded into the previous step's last stage.  Relaxed
+// loads at device scope, which go past the caches: the values come from other
+// XCDs' atomics in earlier kernels
+__device__ __forceinline__ SosIn take_folded(const StepState* st)
 {
-    if (kSosD) atomicExch(&st->sos_bits_d, atomicOr(&st->next_sos_bits_d, 0ull));
-    else       atomicExch(&st->sos_bits, atomicOr(&st->next_sos_bits, 0u));
-    atomicExch(&st->bad_bits, atomicOr(&st->next_bad, 0u));
+    SosIn in;
+    if constexpr (kSosD)
+        in.sos = __longlong_as_double((long long)__hip_atomic_load(&st->next_sos_bits_d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    else
+        in.sos = __uint_as_float(__hip_atomic_load(&st->next_sos_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    in.bad = __hip_atomic_load(&st->next_bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return in;
 }
 
 typedef FaceFluxT<Real> FaceFlux;
@@ -1100,28 +1109,28 @@ struct DtArgs
     double cfl, h, dt_max;
 };
 
-__device__ __forceinline__ void sos_finalize(StepState* st, const DtArgs& d)
+// the finished reduction's targets, put back to zero with its counter
+__device__ __forceinline__ SosIn take_reduction(StepState* st)
 {
-    double sos;
-    if (kSosD) {
-        const unsigned long long bits = atomicOr(&st->sos_bits_d, 0ull);   // coherent read
-        sos = __longlong_as_double((long long)bits);
-        st->sos_d = sos;
-        st->sos = (float)sos;
-        atomicExch(&st->sos_bits_d, 0ull);
-    } else {
-        const float f = __uint_as_float(atomicOr(&st->sos_bits, 0u));
-        sos = f;
-        st->sos = f;
-        st->sos_d = f;
-        atomicExch(&st->sos_bits, 0u);
-    }
+    SosIn in;
+    if constexpr (kSosD) in.sos = __longlong_as_double((long long)atomicExch(&st->sos_bits_d, 0ull));
+    else                 in.sos = __uint_as_float(atomicExch(&st->sos_bits, 0u));
+    in.bad = atomicExch(&st->bad_bits, 0u);
+    atomicExch(&st->sos_count, 0u);
+    return in;
+}
+
+__device__ __forceinline__ void sos_finalize(StepState* st, const DtArgs& d, const SosIn& in)
+{
+    const double sos = in.sos;
+    st->sos_d = sos;
+    st->sos = (float)sos;
     st->sos_is_d = kSosD ? 1 : 0;
-    st->bad = atomicExch(&st->bad_bits, 0u);
+    st->bad = in.bad;
     // the folded maximum (and flag) of the next step starts from zero
-    atomicExch(&st->next_sos_bits, 0u);
-    atomicExch(&st->next_sos_bits_d, 0ull);
-    atomicExch(&st->next_bad, 0u);
+    __hip_atomic_store(&st->next_sos_bits, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&st->next_sos_bits_d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&st->next_bad, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (d.with_dt) {
         // binary64 dt from the binary32 (or binary64) maximum
         double dt = d.cfl*d.h/sos;
@@ -1131,8 +1140,10 @@ __device__ __forceinline__ void sos_finalize(StepState* st, const DtArgs& d)
         st->dtinvh = (float)(dt/d.h);
         st->dtinvh_d = dt/d.h;
     }
-    atomicExch(&st->sos_count, 0u);
 }
+
+// rows a wave of the reduction reads at a time
+constexpr int kSosRows = 4;
 
 // the reduction over the rows of a block, blocks b = 0..nb-1 of it in this
 // launch; returns true in the one thread that finalized (thread (0, 0) of the
@@ -1145,16 +1156,29 @@ __device__ __forceinline__ bool sos_body(const Geom& g, const Real* __restrict__
     const int rows = g.ny * g.nz;
     SosT sos = 0.0f;
     bool bad = false;
-    for (int row = b * 4 + threadIdx.y; row < rows; row += nb * 4) {
-        const int e0 = DENSE ? row * g.nx : g.idx(0, row % g.ny, row / g.ny);
+    // four rows at a time, all their loads in flight; a row past the end
+    // repeats the wave's first one
+    const int step = nb * 4;
+    for (int row = b * 4 + threadIdx.y; row < rows; row += kSosRows * step) {
+        int e0[kSosRows];
+#pragma unroll
+        for (int k = 0; k < kSosRows; ++k) {
+            const int r = row < rows - k * step ? row + k * step : row;
+            e0[k] = DENSE ? r * g.nx : g.idx(0, r % g.ny, r / g.ny);
+        }
         for (int x = threadIdx.x; x < g.nx; x += 64) {
-            const int e = e0 + x;
-            bool cb;
-            const SosT Ec = (kEPair && !DENSE) ? SosT(double(u[4*fs + e]) + double(u[FELO*fs + e]))
-                                               : SosT(u[4*fs + e]);
-            sos = mmax(sos, sos_cell(CPU_FORM != 0, u[e], u[fs + e], u[2*fs + e], u[3*fs + e], Ec,
-                                     u[5*fs + e], u[6*fs + e], cb));
-            bad = bad || cb;
+            Real w[kSosRows][NU];
+#pragma unroll
+            for (int k = 0; k < kSosRows; ++k)
+#pragma unroll
+                for (int q = 0; q < (DENSE ? NVAR : NU); ++q) w[k][q] = u[q*fs + e0[k] + x];
+#pragma unroll
+            for (int k = 0; k < kSosRows; ++k) {
+                bool cb;
+                const SosT Ec = (kEPair && !DENSE) ? SosT(double(w[k][FE]) + double(w[k][NU - 1])) : SosT(w[k][FE]);
+                sos = mmax(sos, sos_cell(CPU_FORM != 0, w[k][0], w[k][1], w[k][2], w[k][3], Ec, w[k][5], w[k][6], cb));
+                bad = bad || cb;
+            }
         }
     }
 #pragma unroll
@@ -1164,13 +1188,16 @@ __device__ __forceinline__ bool sos_body(const Geom& g, const Real* __restrict__
     __syncthreads();
     if (threadIdx.x == 0 && threadIdx.y == 0) {
         const SosT m = mmax(mmax(wmax[0], wmax[1]), mmax(wmax[2], wmax[3]));
-        if (kSosD) atomicMax(&st->sos_bits_d, (unsigned long long)__double_as_longlong((double)m));
-        else       atomicMax(&st->sos_bits, __float_as_uint((float)m));
-        if (wbad[0] | wbad[1] | wbad[2] | wbad[3]) atomicOr(&st->bad_bits, 1u);
-        __threadfence();
+        // Nothing but these atomics passes between the blocks, so they are all
+        // that the count has to follow: the values they return say that they
+        // have been performed.  A device-scope fence here writes back and
+        // invalidates the XCD's L2 once per block (see sos_blocks).
+        unsigned seen = wbad[0] | wbad[1] | wbad[2] | wbad[3] ? atomicOr(&st->bad_bits, 1u) : 0u;
+        if (kSosD) seen += (unsigned)atomicMax(&st->sos_bits_d, (unsigned long long)__double_as_longlong((double)m));
+        else       seen += atomicMax(&st->sos_bits, __float_as_uint((float)m));
+        asm volatile("" : : "v"(seen) : "memory");
         if (atomicAdd(&st->sos_count, 1u) == (unsigned)nb - 1u) {
-            __threadfence();
-            sos_finalize(st, d);
+            sos_finalize(st, d, take_reduction(st));
             return true;
         }
     }
@@ -1181,10 +1208,7 @@ __device__ __forceinline__ bool sos_body(const Geom& g, const Real* __restrict__
 __global__ __launch_bounds__(64)
 void k_sos_folded(StepState* st, const DtArgs d)
 {
-    if (threadIdx.x != 0) return;
-    take_folded(st);
-    __threadfence();
-    sos_finalize(st, d);
+    if (threadIdx.x == 0) sos_finalize(st, d, take_folded(st));
 }
 
 template <int CPU_FORM>
@@ -1410,11 +1434,7 @@ void kb_sos(const BatchDev B, const double cfl, const double dt_max)
     if (C.st->folded) {
         // the previous step's last z sweep folded this state's maximum: only
         // dt remains, done by the case's first block
-        if (local == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
-            take_folded(C.st);
-            __threadfence();
-            sos_finalize(C.st, d);
-        }
+        if (local == 0 && threadIdx.x == 0 && threadIdx.y == 0) sos_finalize(C.st, d, take_folded(C.st));
         return;
     }
     sos_body<CPU_FORM>(C.g, (const Real*)C.u[B.cur[c]], C.g.fstride, C.st, local, C.nb_sos, wmax, wbad, d);
@@ -1652,7 +1672,7 @@ void launch_sos(const Geom& g, const void* uv, StepState* st, const int cpu_form
                 const double h, const double dt_max, hipStream_t s)
 {
     const Real* u = (const Real*)uv;
-    const int nb = rows_grid(g) < 2048 ? rows_grid(g) : 2048;
+    const int nb = mpcf::sos_blocks(g);
     const DtArgs d{with_dt, cfl, h, dt_max};
     if (cpu_form) hipLaunchKernelGGL(k_sos<1>, dim3(nb), dim3(64, 4), 0, s, g, u, g.fstride, st, d);
     else          hipLaunchKernelGGL(k_sos<0>, dim3(nb), dim3(64, 4), 0, s, g, u, g.fstride, st, d);
@@ -1663,8 +1683,7 @@ void launch_sos_dense(const Geom& g, const void* uv, const int64_t fs, StepState
                       int* bad_out, hipStream_t s)
 {
     const Real* u = (const Real*)uv;
-    const int rows = (g.ny * g.nz + 3) / 4;
-    const int nb = rows < 2048 ? rows : 2048;
+    const int nb = mpcf::sos_blocks(g);
     const DtArgs d{1, cfl, h, dt_max};
     if (cpu_form)
         hipLaunchKernelGGL(k_sos_dense<1>, dim3(nb), dim3(64, 4), 0, s, g, u, fs, st, d, sos_out, dt_out, bad_out);
