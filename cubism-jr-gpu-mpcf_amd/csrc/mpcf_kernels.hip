@@ -137,12 +137,14 @@ constexpr int kXCDs = 8;
 // the fused x+y march unrolled by five in the binary32 FAST builds (in the
 // bit-exact and binary64 builds the unrolled march spills)
 constexpr bool kUnrollXY = kFast && !MPCF_F64;
-// the waves of a workgroup of the FAST x+y sweep keep phase (keep_phase)
-// (single-case and batched flat launches: 512^3 step 19.45 -> 18.61 ms, a
-// 24-case ensemble 1.76 -> 1.72 ms; the persistent launches' item loop has
-// barriers of its own that a wave without work reaches early, and does not).
-// The z sweep gains 0.5 % at most and is left alone
-constexpr bool kSyncXY = kFast && !MPCF_F64;
+// the waves of a workgroup of the binary32 x+y sweeps keep phase (keep_phase)
+// (single-case and batched flat launches: FAST 512^3 step 19.45 -> 18.61 ms, a
+// 24-case ensemble 1.76 -> 1.72 ms, bit-exact 256^3 6.58 -> 6.45 ms; the
+// persistent launches' item loop has barriers of its own that a wave without
+// work reaches early, and does not).  The z sweep gains 0.5 % at most and is
+// left alone; a wave that evaluates a window or face again without QUICK does
+// so between two barriers
+constexpr bool kSyncXY = !MPCF_F64;
 // likewise the y / z marches (a separate switch: their register budget differs)
 constexpr bool kUnrollMarch = kFast && !MPCF_F64;
 
@@ -780,7 +782,7 @@ __device__ __forceinline__ RecT<Real> weno_lanes(const Real c, bool* odd)
         keep_phase<SYNC>();
         return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, weno_kD<Real>(Db), weno_kD<Real>(D), weno_kD<Real>(Dd));
     } else {
-        return weno_cell<Real, kFast, QUICK>(from_left(b), b, c, d, from_right(d), odd);
+        return weno_cell<Real, kFast, QUICK, SYNC>(from_left(b), b, c, d, from_right(d), odd);
     }
 }
 template <bool SYNC, bool QUICK>
@@ -788,13 +790,13 @@ __device__ __forceinline__ CellRec reconstruct_lanes_as(const Prim& c, bool* odd
 {
     CellRec o;
     RecT<Real> t;
-    t = weno_lanes<SYNC, QUICK>(c.r, odd); o.m.r = t.m; o.p.r = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.u, odd); o.m.u = t.m; o.p.u = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.v, odd); o.m.v = t.m; o.p.v = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.w, odd); o.m.w = t.m; o.p.w = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.p, odd); o.m.p = t.m; o.p.p = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.G, odd); o.m.G = t.m; o.p.G = t.p;
-    t = weno_lanes<SYNC, QUICK>(c.P, odd); o.m.P = t.m; o.p.P = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.r, odd); o.m.r = t.m; o.p.r = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.u, odd); o.m.u = t.m; o.p.u = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.v, odd); o.m.v = t.m; o.p.v = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.w, odd); o.m.w = t.m; o.p.w = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.p, odd); o.m.p = t.m; o.p.p = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.G, odd); o.m.G = t.m; o.p.G = t.p;
+    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.P, odd); o.m.P = t.m; o.p.P = t.p;
     return o;
 }
 // as reconstruct(): the bit-exact builds take the quick quotients, and the
@@ -853,7 +855,7 @@ struct YRec
     }
     __device__ __forceinline__ CellRec row(const Prim& A, const Prim& B, const Prim& C, const Prim& D, const Prim& E)
     {
-        if constexpr (!kFast) return reconstruct<Real, kFast>(A, B, C, D, E);
+        if constexpr (!kFast) return reconstruct<Real, kFast, SYNC>(A, B, C, D, E);
         CellRec o;
         Rec t;
         t = weno_march<SYNC>(B.r, C.r, D.r, E.r, r); o.m.r = t.m; o.p.r = t.p;

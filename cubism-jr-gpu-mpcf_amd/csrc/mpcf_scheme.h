@@ -309,7 +309,7 @@ MPCF_HD RecT<T> weno_fast_diff(const T b, const T c, const T d, const T dab, con
 // where the product of the indicators (binary32) or of their scaled squares
 // (binary64) is not a normal number, and the caller then evaluates the window
 // again without QUICK
-template <typename T, bool FAST, bool QUICK = false>
+template <typename T, bool FAST, bool QUICK = false, bool SYNC = false>
 MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e, bool* odd = nullptr)
 {
     typedef typename Wide<T>::type W;
@@ -348,6 +348,7 @@ MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e,
             if constexpr (sizeof(T) == 4) *odd = *odd || not_normal(iA*iB*iC);
             else                          *odd = *odd || not_normal(xA*xB*xC);
             rA = rcp_rn(xA); rB = rcp_rn(xB); rC = rcp_rn(xC);
+            keep_phase<SYNC>();
         } else {
             rA = W(1.0) / xA; rB = W(1.0) / xB; rC = W(1.0) / xC;
         }
@@ -367,6 +368,7 @@ MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e,
             T inv;
             if constexpr (QUICK) inv = rcp_rn(sum);
             else                 inv = qdiv<FAST>(T(1.0f), sum);
+            keep_phase<SYNC>();
             const T w0 = pA0 * inv, w1 = pA1 * inv;
             const T w2 = T(1.0f) - w0 - w1;
             out.p = w0*(k1_3*e - k7_6*d + k11_6*c) + w1*(mk1_6*d + k5_6*c + k1_3*b) + w2*(k1_3*c + k5_6*b - k1_6*a);
@@ -383,29 +385,29 @@ MPCF_HD RecT<T> weno_cell(const T a, const T b, const T c, const T d, const T e,
 // one cell's reconstructed face states in one direction
 template <typename T> struct CellRecT { PrimT<T> m, p; };
 
-template <typename T, bool FAST, bool QUICK>
+template <typename T, bool FAST, bool QUICK, bool SYNC = false>
 MPCF_HD CellRecT<T> reconstruct_as(const PrimT<T>& A, const PrimT<T>& B, const PrimT<T>& C, const PrimT<T>& D,
                                    const PrimT<T>& E, bool* odd)
 {
     CellRecT<T> o;
     RecT<T> t;
-    t = weno_cell<T, FAST, QUICK>(A.r, B.r, C.r, D.r, E.r, odd); o.m.r = t.m; o.p.r = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.u, B.u, C.u, D.u, E.u, odd); o.m.u = t.m; o.p.u = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.v, B.v, C.v, D.v, E.v, odd); o.m.v = t.m; o.p.v = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.w, B.w, C.w, D.w, E.w, odd); o.m.w = t.m; o.p.w = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.p, B.p, C.p, D.p, E.p, odd); o.m.p = t.m; o.p.p = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.G, B.G, C.G, D.G, E.G, odd); o.m.G = t.m; o.p.G = t.p;
-    t = weno_cell<T, FAST, QUICK>(A.P, B.P, C.P, D.P, E.P, odd); o.m.P = t.m; o.p.P = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.r, B.r, C.r, D.r, E.r, odd); o.m.r = t.m; o.p.r = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.u, B.u, C.u, D.u, E.u, odd); o.m.u = t.m; o.p.u = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.v, B.v, C.v, D.v, E.v, odd); o.m.v = t.m; o.p.v = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.w, B.w, C.w, D.w, E.w, odd); o.m.w = t.m; o.p.w = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.p, B.p, C.p, D.p, E.p, odd); o.m.p = t.m; o.p.p = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.G, B.G, C.G, D.G, E.G, odd); o.m.G = t.m; o.p.G = t.p;
+    t = weno_cell<T, FAST, QUICK, SYNC>(A.P, B.P, C.P, D.P, E.P, odd); o.m.P = t.m; o.p.P = t.p;
     return o;
 }
 
-template <typename T, bool FAST>
+template <typename T, bool FAST, bool SYNC = false>
 MPCF_HD CellRecT<T> reconstruct(const PrimT<T>& A, const PrimT<T>& B, const PrimT<T>& C, const PrimT<T>& D,
                                 const PrimT<T>& E)
 {
     if constexpr (!FAST && kQuick<T>) {
         bool odd = false;
-        CellRecT<T> o = reconstruct_as<T, FAST, true>(A, B, C, D, E, &odd);
+        CellRecT<T> o = reconstruct_as<T, FAST, true, SYNC>(A, B, C, D, E, &odd);
         if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_as<T, FAST, false>(A, B, C, D, E, nullptr);
         return o;
     } else {
@@ -597,7 +599,7 @@ MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
     if constexpr (!FAST && kQuick<T> && sizeof(T) == 4) {
         bool odd = false;
         FaceFluxT<T> o = riemann_as<D, T, FAST, SYNC, true>(L, Rt, &odd);
-        if (__builtin_expect(any_lane(odd), 0)) o = riemann_as<D, T, FAST, SYNC, false>(L, Rt, nullptr);
+        if (__builtin_expect(any_lane(odd), 0)) o = riemann_as<D, T, FAST, false, false>(L, Rt, nullptr);
         return o;
     } else {
         return riemann_as<D, T, FAST, SYNC, false>(L, Rt, nullptr);
