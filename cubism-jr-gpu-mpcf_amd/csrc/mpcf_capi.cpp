@@ -1166,7 +1166,7 @@ int persist_tables(mpcf_batch* b, std::vector<mpcf::CaseDesc>& desc)
         b->p_cap = cap;
     }
     const int W = b->p_threads / 64;
-    for (mpcf::CaseDesc& d : desc) mpcf::detail::case_items(d, W);
+    for (mpcf::CaseDesc& d : desc) mpcf::detail::case_items(d, W, b->L->xy_tile());
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
     auto cells = [&](int i) { return (long long)desc[i].g.nx * desc[i].g.ny * desc[i].g.nz; };

@@ -70,6 +70,8 @@ struct Launchers
     decltype(&mpcf::parity::batch_z) b_z;
     decltype(&mpcf::parity::persist_stage) persist;
     decltype(&mpcf::parity::persist_occupancy) persist_occ;
+    decltype(&mpcf::parity::xy_tile) xy_tile;
+    decltype(&mpcf::parity::xy_grid) xy_grid;
 };
 
 #define MPCF_LAUNCHERS(NS)                                                                           \
@@ -80,7 +82,7 @@ struct Launchers
      mpcf::NS::launch_test_weno,                                                                      \
      mpcf::NS::launch_test_face,                                                                      \
      mpcf::NS::batch_sos, mpcf::NS::batch_xy, mpcf::NS::batch_z, mpcf::NS::persist_stage,        \
-     mpcf::NS::persist_occupancy}
+     mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid}
 
 inline const Launchers kParity = MPCF_LAUNCHERS(parity);
 inline const Launchers kFast = MPCF_LAUNCHERS(fast);
@@ -233,7 +235,7 @@ inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const 
     d.chunk_xy = len_xy;
     d.chunk_z = std::min(len_z, z_march_limit(c->g));
     int dims[3];
-    parity::xy_grid(c->g, d.chunk_xy, dims);
+    c->L->xy_grid(c->g, d.chunk_xy, dims);
     d.nbx_xy = dims[0]; d.nby_xy = dims[1];
     blocks[0] = dims[0] * dims[1] * dims[2];
     parity::z_grid(c->g, d.chunk_z, dims);
@@ -245,9 +247,9 @@ inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const 
 }
 
 // the persistent stage kernel's items of a case with workgroups of W waves
-inline void case_items(CaseDesc& d, const int W)
+inline void case_items(CaseDesc& d, const int W, const int tile)
 {
-    const int tiles = ((d.g.nx + 6) * d.g.nz + kXYTile - 1) / kXYTile;
+    const int tiles = ((d.g.nx + 6) * d.g.nz + tile - 1) / tile;
     d.wxy = (tiles + W - 1) / W;
     d.items_xy = (unsigned)d.wxy * (unsigned)((d.g.ny + d.chunk_xy - 1) / d.chunk_xy);
     d.wz = (d.g.nx * d.g.ny + 64 * W - 1) / (64 * W);

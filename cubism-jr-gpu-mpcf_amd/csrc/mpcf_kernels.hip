@@ -708,16 +708,28 @@ void k_sweep_x(const Geom g, const StageArgs A, const int chunk)
 
 // ---------------------------------------------------------------------------
 // fused x + y sweep: lanes along x, marching y.  A wave covers 64 consecutive
-// x-cells starting 3 cells left of its tile and writes the 58 cells whose
-// x-stencils lie inside the wave (lanes 3..60); neighbouring tiles overlap by
-// six cells.  The x-direction of row k-1 is computed from the rolling window's
+// x-cells.  FAST: it writes the 58 whose x-stencils lie inside the wave (lanes
+// 3..60), and neighbouring tiles overlap by six cells.  The other builds: it
+// writes the 62 whose faces' two cells lie inside the wave (lanes 1..62); the
+// primitives of two cells beside the wave on either side come from LDS, and
+// neighbouring tiles overlap by two cells.  The x-direction of row k-1 is computed from the rolling window's
 // row k-1 with wave-shifted copies (DPP wave_shr/wave_shl) for the five-point
 // windows, the left face state and the right face flux; the y-direction is
 // the same register march as the y sweep.  The accumulators leave this kernel
 // already summed in the x-then-y order of the reference (GPUkernels.cu:1111),
 // so the x sweep's accumulator round trip disappears.
 // ---------------------------------------------------------------------------
-enum { XY_TILE = kXYTile };
+// The bit-exact and binary64 builds take the two positions beside a wave on
+// either side from LDS and store 62 of its 64 lanes; the FAST builds keep them
+// inside the wave and store 58.  The row's edge values cost FAST 14 differences
+// and the registers of the LDS reads against 6.5 % fewer waves: 512^3 19.4 ms a
+// step against 18.8, 256^3 whole-block 2.69 against 2.60; the bit-exact build,
+// with 3 times the arithmetic per cell, gains: 256^3 6.32 against 6.45, a
+// 600x300x6 block 0.545 against 0.565, binary64 128^3 1.42 against 1.43.
+constexpr bool kHaloLDS = !kFast;
+enum { XY_TILE = kHaloLDS ? 62 : 58 };
+static_assert(!kHaloLDS || !kUnrollXY, "the unrolled march does not refill the rows in LDS");
+constexpr int kHaloRows = 16;   // rows of edge primitives a wave keeps in LDS: 16 x 4 positions fill its lanes
 
 // value of lane l-1 / lane l+1.  The wave's edge lanes (no source lane) read
 // zero: they are halo positions whose results are never stored, and with no
@@ -741,6 +753,29 @@ __device__ __forceinline__ double dpp_move(const double v)
 }
 __device__ __forceinline__ Real from_left(const Real v) { return dpp_move<0x138>(v); }    // wave_shr:1
 __device__ __forceinline__ Real from_right(const Real v) { return dpp_move<0x130>(v); }   // wave_shl:1
+// the same, the wave's edge lane taking `edge` (its value in that lane)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(const float edge, const float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, v),
+                                                                 CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(const double edge, const double v)
+{
+    const long long b = __builtin_bit_cast(long long, v), o = __builtin_bit_cast(long long, edge);
+    const int lo = __builtin_amdgcn_update_dpp((int)(o & 0xffffffffLL), (int)(b & 0xffffffffLL), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ __forceinline__ Real from_left(const Real edge, const Real v) { return dpp_move<0x138>(edge, v); }
+__device__ __forceinline__ Real from_right(const Real edge, const Real v) { return dpp_move<0x130>(edge, v); }
+
+// One primitive at the four positions beside a wave, as the x reconstruction
+// of its edge lanes needs it: two and one left of lane 0, one and two right of
+// lane 63 (kHaloLDS)
+typedef Real Halo4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ Prim prim_from_left(const Prim& q)
 {
     Prim o;
@@ -759,7 +794,7 @@ __device__ __forceinline__ Prim prim_from_right(const Prim& q)
 // workgroups go to the XCDs round-robin by linear id; this maps linear id
 // `lin` of a grid of n to a tile index such that each XCD takes a contiguous
 // run of tiles, so that neighbouring tiles of the fused x+y sweep (which
-// overlap by six positions and share partial cache lines) meet in one L2.
+// overlap by two positions and share partial cache lines) meet in one L2.
 // For grids of equal-cost tiles (one block)
 __device__ __forceinline__ int xcd_order(const int lin, const int n)
 {
@@ -768,49 +803,53 @@ __device__ __forceinline__ int xcd_order(const int lin, const int n)
     return xcd * per + min(xcd, extra) + k;
 }
 
-// x-direction reconstruction of each lane's cell from its lane neighbours.
+// x-direction reconstruction of each lane's cell from its lane neighbours (and,
+// kHaloLDS, at the wave's edges the positions beside it).
 // FAST: the second difference is formed once per lane and shifted (a lane's Db
 // is its left neighbour's Dc, the same subtractions of the same values)
 template <bool SYNC, bool QUICK>
-__device__ __forceinline__ RecT<Real> weno_lanes(const Real c, bool* odd)
+__device__ __forceinline__ RecT<Real> weno_lanes(const Real c, const Halo4 h, bool* odd)
 {
-    const Real b = from_left(c), d = from_right(c);
     if constexpr (kFast) {
+        const Real b = from_left(c), d = from_right(c);
         const Real dbc = c - b, dcd = d - c;
         const Real D = dcd - dbc;
         const Real Db = from_left(D), Dd = from_right(D);
         keep_phase<SYNC>();
         return weno_fast_core<Real, SYNC>(b, c, d, dbc, dcd, Db, D, Dd, weno_kD<Real>(Db), weno_kD<Real>(D), weno_kD<Real>(Dd));
     } else {
-        return weno_cell<Real, kFast, QUICK, SYNC>(from_left(b), b, c, d, from_right(d), odd);
+        const Real b = from_left(h[1], c), d = from_right(h[2], c);
+        return weno_cell<Real, kFast, QUICK, SYNC>(from_left(h[0], b), b, c, d, from_right(h[3], d), odd);
     }
 }
+// halo: the row's Halo4 of the seven primitives
 template <bool SYNC, bool QUICK>
-__device__ __forceinline__ CellRec reconstruct_lanes_as(const Prim& c, bool* odd)
+__device__ __forceinline__ CellRec reconstruct_lanes_as(const Prim& c, const Halo4* halo, bool* odd)
 {
+    constexpr bool S = SYNC && (kFast || QUICK);
     CellRec o;
     RecT<Real> t;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.r, odd); o.m.r = t.m; o.p.r = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.u, odd); o.m.u = t.m; o.p.u = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.v, odd); o.m.v = t.m; o.p.v = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.w, odd); o.m.w = t.m; o.p.w = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.p, odd); o.m.p = t.m; o.p.p = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.G, odd); o.m.G = t.m; o.p.G = t.p;
-    t = weno_lanes<SYNC && (kFast || QUICK), QUICK>(c.P, odd); o.m.P = t.m; o.p.P = t.p;
+    t = weno_lanes<S, QUICK>(c.r, halo[0], odd); o.m.r = t.m; o.p.r = t.p;
+    t = weno_lanes<S, QUICK>(c.u, halo[1], odd); o.m.u = t.m; o.p.u = t.p;
+    t = weno_lanes<S, QUICK>(c.v, halo[2], odd); o.m.v = t.m; o.p.v = t.p;
+    t = weno_lanes<S, QUICK>(c.w, halo[3], odd); o.m.w = t.m; o.p.w = t.p;
+    t = weno_lanes<S, QUICK>(c.p, halo[4], odd); o.m.p = t.m; o.p.p = t.p;
+    t = weno_lanes<S, QUICK>(c.G, halo[5], odd); o.m.G = t.m; o.p.G = t.p;
+    t = weno_lanes<S, QUICK>(c.P, halo[6], odd); o.m.P = t.m; o.p.P = t.p;
     return o;
 }
 // as reconstruct(): the bit-exact builds take the quick quotients, and the
 // IEEE ones where a lane's window needs them
 template <bool SYNC>
-__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c)
+__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c, const Halo4* halo)
 {
     if constexpr (!kFast) {
         bool odd = false;
-        CellRec o = reconstruct_lanes_as<SYNC, true>(c, &odd);
-        if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_lanes_as<SYNC, false>(c, nullptr);
+        CellRec o = reconstruct_lanes_as<SYNC, true>(c, halo, &odd);
+        if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_lanes_as<SYNC, false>(c, halo, nullptr);
         return o;
     } else {
-        return reconstruct_lanes_as<SYNC, false>(c, nullptr);
+        return reconstruct_lanes_as<SYNC, false>(c, halo, nullptr);
     }
 }
 
@@ -876,19 +915,25 @@ struct YRec
 // rows of the same chunk, and a wave past the end leaves the kernel
 template <bool FIRST = false, bool SYNC = false>
 __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A, const int chunk,
-                                              const int wv, const int bz)
+                                              const int wv, const int wib, const int bz)
 {
     // positions q along the padded rows (x = -3 .. nx+2) of all z-planes,
-    // flattened; wave w covers q = 58 w .. 58 w + 63 and stores lanes 3..60,
-    // so consecutive waves overlap by six positions and ghost positions are
-    // computed but never stored
+    // flattened; ghost positions are computed but never stored.  Wave w (wib:
+    // its place in the workgroup) of the FAST builds covers q = 58 w .. 58 w +
+    // 63 and stores lanes 3..60, so consecutive waves overlap by six positions.
+    // kHaloLDS: it covers q = 62 w + 2 .. 62 w + 65 and stores lanes 1..62: a
+    // stored cell's faces need the reconstruction of its lane neighbours, and
+    // theirs the primitives of two positions beside the wave on either side.
+    // Those come from LDS, where the wave puts them for 16 rows at a time, a
+    // lane per row and position (one conversion of 64 lanes, then 7 broadcast
+    // reads a row), bit for bit what the neighbouring wave computes.
     const int lane = threadIdx.x & 63;
     const int rowlen = g.nx + 6;
     const int nzr = A.z1 - A.z0;                  // planes of this launch
-    const int q = wv * XY_TILE + lane;
+    const int q = wv * XY_TILE + (kHaloLDS ? 2 : 0) + lane;
     int z = q / rowlen;
     const int x = q - z * rowlen - 3;
-    const bool store = lane >= 3 && lane <= 60 && x >= 0 && x < g.nx && z < nzr;
+    const bool store = lane >= (kHaloLDS ? 1 : 3) && lane <= (kHaloLDS ? 62 : 60) && x >= 0 && x < g.nx && z < nzr;
     if (wv * XY_TILE >= rowlen * nzr) return;     // whole wave past the end
     z = A.z0 + min(z, nzr - 1);                   // lanes past the last plane read its last row
     // lanes outside [0, nx) read the cell their x-ghost copies
@@ -914,6 +959,32 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
     auto fix = [&](Real* o, const Real sgy) {
         o[FV] *= sgy;
         if (xmirror) o[FU] *= sgx;
+    };
+
+    __shared__ Halo4 sh_halo[kHaloLDS ? 4 : 1][kHaloLDS ? kHaloRows : 1][NVAR];
+    // primitives beside the wave of rows [h0, h0 + kHaloRows), interior rows
+    int h0 = c0 - kHaloRows;
+    auto fill_halo = [&](const int row0) {
+        h0 = row0;
+        const int j = lane >> 2, side = lane & 3;
+        const int row = min(row0 + j, c1 - 1);
+        // a position left of the wave's first plane is never needed (it reads
+        // that plane's first ghost)
+        const int qh = max(wv * XY_TILE + (side < 2 ? side : 64 + side), (wv * XY_TILE + 2) / rowlen * rowlen);
+        const int zq = qh / rowlen;
+        Real sx;
+        const int xh = bc_index(qh - zq * rowlen - 3, g.nx, A.bcmask, 0, sx);
+        const uint32_t off = (uint32_t)(g.idx(xh, row, A.z0 + min(zq, nzr - 1)) - L.base) * (uint32_t)sizeof(Real);
+        Real w[NU];
+#pragma unroll
+        for (int f = 0; f < NU; ++f) w[f] = ld_lane(U.p[f], off);
+        if (xmirror) w[FU] *= sx;
+        const Prim p = prim_of(w);
+        const Real v[NVAR] = {p.r, p.u, p.v, p.w, p.p, p.G, p.P};
+#pragma unroll
+        for (int f = 0; f < NVAR; ++f) {
+            sh_halo[wib][j][f][side] = v[f];
+        }
     };
 
     March<1, MODE_ACC> m;
@@ -950,7 +1021,11 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
             const FaceFlux Fy = riemann<1, Real, kFast, SYNC>(m.pm, ry.p);          // face k-1/2
             if (EMIT) {
                 // x-direction of row k-1 (window slot w1)
-                const CellRec rx = reconstruct_lanes<SYNC>(m.w1);
+                Halo4 halo[NVAR];
+#pragma unroll
+                for (int f = 0; f < NVAR; ++f)
+                    if constexpr (kHaloLDS) halo[f] = sh_halo[wib][k - 1 - h0][f];
+                const CellRec rx = reconstruct_lanes<SYNC>(m.w1, halo);
                 const Prim Lm = prim_from_left(rx.m);
                 const FaceFlux Fxl = riemann<0, Real, kFast, SYNC>(Lm, rx.p);      // face x-1/2
                 FaceFlux Fxr;                                                        // face x+1/2
@@ -993,7 +1068,10 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
         for (; k < c1; ++k) step(T_{}, T_{}, T_{}, k);
         step(T_{}, T_{}, F_{}, c1);      // c1 >= c0 + 1: every chunk has a row
     } else {
-        for (int k = c0 - 1; k <= c1; ++k) step(k >= c0, k >= c0 + 1, k < c1, k);
+        for (int k = c0 - 1; k <= c1; ++k) {
+            if (kHaloLDS && k > c0 && k > h0 + kHaloRows) fill_halo(k - 1);
+            step(k >= c0, k >= c0 + 1, k < c1, k);
+        }
     }
 }
 
@@ -1014,7 +1092,7 @@ void k_sweep_xy(const Geom g, const StageArgs A, const int chunk)
     __builtin_amdgcn_s_setprio(2);
     const int gx = gridDim.x;
     const int t = xcd_order(blockIdx.x + blockIdx.y * gx, gx * gridDim.y);
-    sweep_xy_body<FIRST, kSyncXY>(g, A, chunk, (t % gx) * 4 + threadIdx.y, t / gx);
+    sweep_xy_body<FIRST, kSyncXY>(g, A, chunk, (t % gx) * 4 + threadIdx.y, threadIdx.y, t / gx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1453,7 +1531,7 @@ void kb_sweep_xy(const BatchDev B, const Real a, const Real b)
     const CaseDesc& C = B.cases[c];
     const int local = blockIdx.x - B.off_xy[c];
     const StageArgs A = case_args(C, B.cur[c], a, b);
-    sweep_xy_body<FIRST, kSyncXY>(C.g, A, C.chunk_xy, (local % C.nbx_xy) * 4 + threadIdx.y, local / C.nbx_xy);
+    sweep_xy_body<FIRST, kSyncXY>(C.g, A, C.chunk_xy, (local % C.nbx_xy) * 4 + threadIdx.y, threadIdx.y, local / C.nbx_xy);
 }
 
 // the z sweep finishes the stage; the last block of each case to finish
@@ -1493,7 +1571,7 @@ void kb_sweep_z(const BatchDev B, const Real a, const Real b, const int fold, co
 // which measured 1.7x slower than flat launches).  Each workgroup pulls items
 // from a device queue (an atomic counter) until it is empty; an item is one
 // workgroup's share of one case's x+y sweep (W = blockDim.x / 64 consecutive
-// 58-position tiles over one y-chunk) or z sweep (blockDim.x columns over one
+// 62-position tiles over one y-chunk) or z sweep (blockDim.x columns over one
 // z-chunk), running the single-case bodies, so every case gets exactly the
 // arithmetic it gets alone.  The queue holds the items of the larger cases
 // first, so the small ones fill the launch's tail.
@@ -1557,7 +1635,7 @@ __device__ __forceinline__ void kp_stage_body(const PersistDev& P, const Real a,
         StageArgs A = case_args(C, cur, a, b);
         if constexpr (phase == 0) {
             (void)fold; (void)cpu_form;
-            sweep_xy_body(C.g, A, C.chunk_xy, (j % C.wxy) * W + wib, j / C.wxy);
+            sweep_xy_body(C.g, A, C.chunk_xy, (j % C.wxy) * W + wib, wib, j / C.wxy);
         } else {
             if (fold) { A.sos_next = C.st; A.sos_cpu = cpu_form; }
             sweep_yz_body<2, MODE_STAGE>(C.g, A, C.chunk_z, (j % C.wz) * (int)blockDim.x + (int)threadIdx.x, j / C.wz);
@@ -1807,6 +1885,9 @@ int whole_chunk(const Geom& g, const int dir)
 {
     return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3) : whole_march(g.nz, z_blocks(g), 2);
 }
+
+// positions a wave of the fused x+y sweep stores
+int xy_tile() { return XY_TILE; }
 
 // grid of the fused x+y sweep: dims[0] blocks of four waves over the padded
 // rows of all planes, dims[2] y-chunks (dims[1] = 1)

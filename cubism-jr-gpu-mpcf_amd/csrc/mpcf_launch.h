@@ -9,10 +9,6 @@
 #include "mpcf_geom.h"
 
 namespace mpcf {
-// positions of a wave of the fused x+y sweep that it stores (64 lanes less
-// the three-cell x-halo on each side)
-constexpr int kXYTile = 58;
-
 // arguments of one direction sweep of a stage
 struct SweepParams
 {
@@ -118,6 +114,7 @@ void batch_z(const BatchDev& B, int blocks, double a, double b, int fold, int cp
 void persist_stage(const PersistDev& P, const int blocks[2], int threads, double a, double b, int fold,     \
                    int cpu_form, hipStream_t s);                                                           \
 int persist_occupancy(int threads, int phase);                                                             \
+int xy_tile();                                                                                             \
 void xy_grid(const Geom& g, int chunk, int dims[3]);                                                       \
 void z_grid(const Geom& g, int chunk, int dims[3]);                                                        \
 int whole_chunk(const Geom& g, int dir);                                                                   \
