@@ -79,17 +79,50 @@ typedef std::conditional<kSosD, double, float>::type SosT;
 // a P negative enough to matter drives c^2 <= 0, which is flagged.  Every comparison is false for a NaN, and a NaN
 // in any field reaches p and c, so a NaN cell is always flagged -- the maximum
 // itself drops NaN operands (fmax) and would not show it.
-__device__ __forceinline__ SosT sos_cell(const bool cpu_form, const SosT r, const SosT mu, const SosT mv,
-                                         const SosT mw, const SosT E, const SosT G, const SosT P, bool& bad)
+// QUICK (binary32, GPU form): the quotients and the root by div_rn and sqrt_rn,
+// which round like the IEEE operations; `odd` is set where an operand is
+// outside [2^-40, 2^40] (all but the momentum's quotient, which a momentum too
+// small for div_rn leaves without effect on the sum), and sos_cell then
+// evaluates the cell again without QUICK.  29 instructions instead of 72.
+template <bool QUICK>
+__device__ __forceinline__ SosT sos_cell_as(const bool cpu_form, const SosT r, const SosT mu, const SosT mv,
+                                            const SosT mw, const SosT E, const SosT G, const SosT P, bool& bad, bool* odd)
 {
-    SosT p;
-    if (cpu_form) p = (SosT)((E - (mu*mu + mv*mv + mw*mw)*(0.5/r) - P)/G);
-    else          p = (E - (mu*mu + mv*mv + mw*mw)*(SosT(0.5f)/r) - P) / G;
-    const SosT c = msqrt(((p + P) / G + p) / r);
-    const SosT s = c + mmax(mmax(fabs(mu), fabs(mv)), fabs(mw)) / r;
+    SosT c, s;
+    const SosT mm = mmax(mmax(fabs(mu), fabs(mv)), fabs(mw));
+    if constexpr (QUICK) {
+        const SosT ir = rcp_rn(r), iG = rcp_rn(G);
+        const SosT p = div_rn(E - (mu*mu + mv*mv + mw*mw)*div_rn(SosT(0.5f), r, ir) - P, G, iG);
+        const SosT x = div_rn(p + P, G, iG) + p;
+        const SosT c2 = div_rn(x, r, ir);
+        c = sqrt_rn(c2);
+        s = c + div_rn(mm, r, ir);
+        const SosT lo = mmin3(mmin3(r, G, p + P), mmin3(x, c2, fabs(p)), fabs(p));
+        const SosT hi = mmax3(mmax3(r, G, p + P), mmax3(x, c2, fabs(p)), mm);
+        *odd = !(lo >= SosT(0x1p-40f) && hi <= SosT(0x1p40f));
+    } else {
+        SosT p;
+        if (cpu_form) p = (SosT)((E - (mu*mu + mv*mv + mw*mw)*(0.5/r) - P)/G);
+        else          p = (E - (mu*mu + mv*mv + mw*mw)*(SosT(0.5f)/r) - P) / G;
+        c = msqrt(((p + P) / G + p) / r);
+        s = c + mm / r;
+    }
     const SosT huge = kSosD ? SosT(__DBL_MAX__) : SosT(__FLT_MAX__);
     bad = !(r > SosT(0) && E > SosT(0) && G > SosT(0) && c > SosT(0) && s <= huge);
     return s;
+}
+
+__device__ __forceinline__ SosT sos_cell(const bool cpu_form, const SosT r, const SosT mu, const SosT mv,
+                                         const SosT mw, const SosT E, const SosT G, const SosT P, bool& bad)
+{
+    if constexpr (!kSosD) {
+        bool odd = cpu_form;
+        if (!cpu_form) {
+            const SosT s = sos_cell_as<true>(false, r, mu, mv, mw, E, G, P, bad, &odd);
+            if (__builtin_expect(!any_lane(odd), 1)) return s;
+        }
+    }
+    return sos_cell_as<false>(cpu_form, r, mu, mv, mw, E, G, P, bad, nullptr);
 }
 
 // a maximum speed of sound and its flag as a reduction or a step's last stage
@@ -562,8 +595,11 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
 
 // column `col` of the columns (x, t) flattened x-fastest: consecutive lanes
 // are consecutive x (coalesced) and no lane idles when nx is not a multiple
-// of 64.  Every lane of the wave takes part (the fold reduction is per wave)
-template <int D, int MODE>
+// of 64.  Every thread of the workgroup (256 threads, unless PER_WAVE) takes
+// part (the fold reduction)
+// PER_WAVE: the fold's atomics are issued by every wave, with no barrier (the
+// persistent kernels, whose item loop keeps its barriers in calls of their own)
+template <int D, int MODE, bool PER_WAVE = false>
 __device__ __forceinline__ void sweep_yz_body(const Geom& g, const StageArgs& A, const int chunk,
                                               const int col, const int bz)
 {
@@ -572,17 +608,29 @@ __device__ __forceinline__ void sweep_yz_body(const Geom& g, const StageArgs& A,
     bool bad = false;
     if (col < g.nx * nt) smax = sweep_yz_column<D, MODE>(g, A, chunk, col, bz, bad);   // no barriers in the body
     if (is_stage(MODE) && A.sos_next) {
-        // one atomic max (and, for a bad cell, one atomic or) per wave; every
-        // lane of the wave takes part
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) smax = mmax(smax, __shfl_xor(smax, off, 64));
-        const bool wbad = __ballot(bad) != 0;
-        if ((threadIdx.x & 63) == 0) {
+        int anybad = __ballot(bad) != 0;
+        const int wave = threadIdx.x >> 6;
+        bool first = (threadIdx.x & 63) == 0;
+        if constexpr (!PER_WAVE) {
+            // one atomic max (and, for a bad cell, one atomic or) per workgroup:
+            // they take turns at one address, and one per wave took 5 us of
+            // the 12 us of a 32^3 block's last sweep
+            __shared__ SosT wmax[4];
+            __shared__ int wbad[4];
+            if (first) { wmax[wave] = smax; wbad[wave] = anybad; }
+            __syncthreads();
+            smax = mmax(mmax(wmax[0], wmax[1]), mmax(wmax[2], wmax[3]));
+            anybad = wbad[0] | wbad[1] | wbad[2] | wbad[3];
+            first = threadIdx.x == 0;
+        }
+        if (first) {
             if (smax > SosT(0)) {
                 if (kSosD) atomicMax(&A.sos_next->next_sos_bits_d, (unsigned long long)__double_as_longlong((double)smax));
                 else       atomicMax(&A.sos_next->next_sos_bits, __float_as_uint((float)smax));
             }
-            if (wbad) atomicOr(&A.sos_next->next_bad, 1u);
+            if (anybad) atomicOr(&A.sos_next->next_bad, 1u);
         }
     }
 }
@@ -1638,7 +1686,7 @@ __device__ __forceinline__ void kp_stage_body(const PersistDev& P, const Real a,
             sweep_xy_body(C.g, A, C.chunk_xy, (j % C.wxy) * W + wib, wib, j / C.wxy);
         } else {
             if (fold) { A.sos_next = C.st; A.sos_cpu = cpu_form; }
-            sweep_yz_body<2, MODE_STAGE>(C.g, A, C.chunk_z, (j % C.wz) * (int)blockDim.x + (int)threadIdx.x, j / C.wz);
+            sweep_yz_body<2, MODE_STAGE, true>(C.g, A, C.chunk_z, (j % C.wz) * (int)blockDim.x + (int)threadIdx.x, j / C.wz);
             count_z(P.done + S.c, C.items_z, &P.cur[S.c], cur, &C.st->folded, fold);
         }
     }

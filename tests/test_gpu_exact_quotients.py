@@ -75,3 +75,26 @@ def test_faces_every_magnitude(mpcf, oracle, kind, d):
     with np.errstate(over="ignore", under="ignore"):
         st = np.ascontiguousarray(st.astype(np.float32))
     equal(mpcf.test_face(st, d), oracle.face_batch(st, d), "face")
+
+
+@pytest.mark.parametrize("kind", ["usual", "scaled", "fading"])
+def test_speed_of_sound_every_magnitude(mpcf, oracle, kind):
+    """small blocks of one state each, so that the maximum is that state's"""
+    rng = np.random.default_rng(3)
+    print("[quotients] sos", kind, flush=True)
+    n = (5, 6, 7)
+    for i in range(60):
+        mag = (lambda: 10.0 ** rng.uniform(-14, 13)) if kind == "scaled" else (lambda: 10.0 ** rng.uniform(-1, 3))
+        rho, p, G, P = mag(), mag(), mag() * (1 if kind == "scaled" else 1e-2), mag()
+        m = rng.uniform(-1, 1, 3) * (10.0 ** rng.uniform(-45, -8) if kind == "fading" else np.sqrt(rho * p))
+        E = G * p + P + 0.5 * (m ** 2).sum() / rho
+        s = np.empty((7,) + n[::-1], np.float32)
+        s[:] = np.array([rho, *m, E, G, P], np.float64).astype(np.float32)[:, None, None, None]
+        ob = oracle.Block(*n)
+        ob.data = s
+        ref = ob.max_sos(False)
+        if not np.isfinite(ref) or not ref > 0:
+            continue
+        with mpcf.Block(*n, 0.1) as b:
+            b.data = s
+            assert b.max_sos() == ref, (i, rho, p, G, P, m)
