@@ -1221,7 +1221,7 @@ int batch_rebuild(mpcf_batch* b)
     std::vector<mpcf::CaseDesc> desc(n);
     const int tab = 3 * (b->cap + 1);
     std::vector<int> cur(n), off(kBatchGroups * tab, 0);
-    long long cols_xy = 0, cols_z = 0;
+    long long cols_xy = 0, cols_z = 0, cells = 0;
     for (mpcf_ctx* c : b->cases) {
         cols_xy += (long long)(c->g.nx + 6) * c->g.nz;
         cols_z += (long long)c->g.nx * c->g.ny;
@@ -1229,7 +1229,7 @@ int batch_rebuild(mpcf_batch* b)
     int first[kBatchGroups + 1];
     {
         std::vector<long long> cc(n);
-        for (int i = 0; i < n; ++i) cc[i] = (long long)b->cases[i]->g.nx * b->cases[i]->g.ny * b->cases[i]->g.nz;
+        for (int i = 0; i < n; ++i) cells += cc[i] = (long long)b->cases[i]->g.nx * b->cases[i]->g.ny * b->cases[i]->g.nz;
         split_groups(cc.data(), n, kBatchGroups, first);
     }
     for (int i = 0; i < n; ++i) {
@@ -1242,7 +1242,7 @@ int batch_rebuild(mpcf_batch* b)
         int* os = oxy + 2 * (b->cap + 1);
         int blocks[3];
         mpcf::detail::case_desc(c, c->cur, march_len(b, i, c->g.ny, 0, cols_xy), march_len(b, i, c->g.nz, 1, cols_z),
-                                desc[i], blocks);
+                                cells, desc[i], blocks);
         oxy[j + 1] = oxy[j] + blocks[0];
         oz[j + 1] = oz[j] + blocks[1];
         os[j + 1] = os[j] + blocks[2];

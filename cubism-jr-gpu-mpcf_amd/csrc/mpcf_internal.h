@@ -72,6 +72,7 @@ struct Launchers
     decltype(&mpcf::parity::persist_occupancy) persist_occ;
     decltype(&mpcf::parity::xy_tile) xy_tile;
     decltype(&mpcf::parity::xy_grid) xy_grid;
+    decltype(&mpcf::parity::z_width) z_width;
 };
 
 #define MPCF_LAUNCHERS(NS)                                                                           \
@@ -82,7 +83,7 @@ struct Launchers
      mpcf::NS::launch_test_weno,                                                                      \
      mpcf::NS::launch_test_face,                                                                      \
      mpcf::NS::batch_sos, mpcf::NS::batch_xy, mpcf::NS::batch_z, mpcf::NS::persist_stage,        \
-     mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid}
+     mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid, mpcf::NS::z_width}
 
 inline const Launchers kParity = MPCF_LAUNCHERS(parity);
 inline const Launchers kFast = MPCF_LAUNCHERS(fast);
@@ -226,8 +227,10 @@ inline int batch_march(const int nd, const int forced, const int tuned)
 }
 
 // descriptor of one case for the batch kernels, and its block counts in the
-// flat grids: blocks[0] x+y sweep, [1] z sweep, [2] speed of sound
-inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const int len_z, CaseDesc& d, int blocks[3])
+// flat grids: blocks[0] x+y sweep, [1] z sweep, [2] speed of sound.  `cells`: of
+// all cases that step together
+inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const int len_z, const long long cells,
+                      CaseDesc& d, int blocks[3])
 {
     d.g = c->g;
     d.u[0] = c->u[0]; d.u[1] = c->u[1]; d.R = c->R; d.acc = c->acc; d.st = c->st; d.h = c->h;
@@ -238,7 +241,8 @@ inline void case_desc(const mpcf_ctx* c, const int cur, const int len_xy, const 
     c->L->xy_grid(c->g, d.chunk_xy, dims);
     d.nbx_xy = dims[0]; d.nby_xy = dims[1];
     blocks[0] = dims[0] * dims[1] * dims[2];
-    parity::z_grid(c->g, d.chunk_z, dims);
+    d.width_z = c->L->z_width(c->g.nx, cells);
+    parity::z_grid(c->g, d.width_z, d.chunk_z, dims);
     d.nbx_z = dims[0]; d.nby_z = dims[1];
     blocks[1] = dims[0] * dims[1] * dims[2];
     d.nb_sos = sos_blocks(c->g);
@@ -252,7 +256,7 @@ inline void case_items(CaseDesc& d, const int W, const int tile)
     const int tiles = ((d.g.nx + 6) * d.g.nz + tile - 1) / tile;
     d.wxy = (tiles + W - 1) / W;
     d.items_xy = (unsigned)d.wxy * (unsigned)((d.g.ny + d.chunk_xy - 1) / d.chunk_xy);
-    d.wz = (d.g.nx * d.g.ny + 64 * W - 1) / (64 * W);
+    d.wz = (d.width_z * d.g.ny + 64 * W - 1) / (64 * W);
     d.items_z = (unsigned)d.wz * (unsigned)((d.g.nz + d.chunk_z - 1) / d.chunk_z);
 }
 

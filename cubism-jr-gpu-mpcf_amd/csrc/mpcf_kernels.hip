@@ -503,15 +503,14 @@ __device__ __forceinline__ Real stage_dtinvh(const StageArgs& A)
 // cells it wrote and sets bad if one of them is non-finite or non-physical
 // (zero / false unless A.sos_next)
 template <int D, int MODE>
-__device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& A, const int chunk, const int col,
-                                                const int bz, bool& bad)
+__device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& A, const int chunk, const int x,
+                                                const int row, const int bz, bool& bad)
 {
     const int nd = D == 1 ? g.ny : g.nz;
-    const int x = col % g.nx;
     // the y sweep's columns lie in the launch's planes [z0, z1); the z sweep
     // marches its launch's rows [z0, z1) (boundary conditions still use the
     // whole extent nd)
-    const int t = (D == 1 ? A.z0 : 0) + col / g.nx;
+    const int t = (D == 1 ? A.z0 : 0) + row;
     const int c0 = (D == 2 ? A.z0 : 0) + bz * chunk;
     const int c1 = min(c0 + chunk, D == 2 ? A.z1 : nd);
     const int s = g.stride(D);
@@ -593,20 +592,21 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
     return m.smax;
 }
 
-// column `col` of the columns (x, t) flattened x-fastest: consecutive lanes
-// are consecutive x (coalesced) and no lane idles when nx is not a multiple
-// of 64.  Every thread of the workgroup (256 threads, unless PER_WAVE) takes
+// column `col` of the columns (x, t) flattened x-fastest, `width` of them a row
+// (nx, or z_width's for a z sweep): consecutive lanes are consecutive x
+// (coalesced); the columns x >= nx idle.  Every thread of the workgroup (256 threads, unless PER_WAVE) takes
 // part (the fold reduction)
 // PER_WAVE: the fold's atomics are issued by every wave, with no barrier (the
 // persistent kernels, whose item loop keeps its barriers in calls of their own)
 template <int D, int MODE, bool PER_WAVE = false>
 __device__ __forceinline__ void sweep_yz_body(const Geom& g, const StageArgs& A, const int chunk,
-                                              const int col, const int bz)
+                                              const int width, const int col, const int bz)
 {
     const int nt = D == 1 ? A.z1 - A.z0 : g.ny;
     SosT smax = 0;
     bool bad = false;
-    if (col < g.nx * nt) smax = sweep_yz_column<D, MODE>(g, A, chunk, col, bz, bad);   // no barriers in the body
+    const int row = col / width, x = col - row * width;
+    if (row < nt && x < g.nx) smax = sweep_yz_column<D, MODE>(g, A, chunk, x, row, bz, bad);   // no barriers in the body
     if (is_stage(MODE) && A.sos_next) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) smax = mmax(smax, __shfl_xor(smax, off, 64));
@@ -637,9 +637,9 @@ __device__ __forceinline__ void sweep_yz_body(const Geom& g, const StageArgs& A,
 
 template <int D, int MODE>
 __global__ __launch_bounds__(256)
-void k_sweep_yz(const Geom g, const StageArgs A, const int chunk)
+void k_sweep_yz(const Geom g, const StageArgs A, const int chunk, const int width)
 {
-    sweep_yz_body<D, MODE>(g, A, chunk, blockIdx.x * 256 + threadIdx.x, blockIdx.y);
+    sweep_yz_body<D, MODE>(g, A, chunk, width, blockIdx.x * 256 + threadIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1598,7 +1598,7 @@ void kb_sweep_z(const BatchDev B, const Real a, const Real b, const int fold, co
     const int local = blockIdx.x - B.off_z[c];
     StageArgs A = case_args(C, B.cur[c], a, b);
     if (fold) { A.sos_next = C.st; A.sos_cpu = cpu_form; }
-    sweep_yz_body<2, MODE>(C.g, A, C.chunk_z, (local % C.nbx_z) * 256 + threadIdx.x, local / C.nbx_z);
+    sweep_yz_body<2, MODE>(C.g, A, C.chunk_z, C.width_z, (local % C.nbx_z) * 256 + threadIdx.x, local / C.nbx_z);
     __syncthreads();
     if (threadIdx.x == 0) {
         const unsigned nblk = (unsigned)(B.off_z[c + 1] - B.off_z[c]);
@@ -1686,7 +1686,7 @@ __device__ __forceinline__ void kp_stage_body(const PersistDev& P, const Real a,
             sweep_xy_body(C.g, A, C.chunk_xy, (j % C.wxy) * W + wib, wib, j / C.wxy);
         } else {
             if (fold) { A.sos_next = C.st; A.sos_cpu = cpu_form; }
-            sweep_yz_body<2, MODE_STAGE, true>(C.g, A, C.chunk_z, (j % C.wz) * (int)blockDim.x + (int)threadIdx.x, j / C.wz);
+            sweep_yz_body<2, MODE_STAGE, true>(C.g, A, C.chunk_z, C.width_z, (j % C.wz) * (int)blockDim.x + (int)threadIdx.x, j / C.wz);
             count_z(P.done + S.c, C.items_z, &P.cur[S.c], cur, &C.st->folded, fold);
         }
     }
@@ -1756,14 +1756,32 @@ static int whole_march(const int nd, const int64_t blocks, const int dir)
     return best;
 }
 
+// columns of a z sweep's rows of nx, in a launch (or a batch's launches) over
+// `cells` cells.  The FAST builds' z sweep runs at the memory's rate: rows
+// rounded up to 32 columns give every half wave one whole 128-byte line a
+// field, where the packed columns of an odd nx read and write each line in
+// parts, from two waves.  Smaller blocks stay in the L2s and only feel the idle
+// lanes, and the EPAIR build (eight fields and more arithmetic) gains later.  Measured,
+// packed / rounded z sweep, us: 80^3 22.2 / 23.8, 90^3 28.2 / 26.4, 129x64x64
+// 24.7 / 23.6, 97^3 37.5 / 34.6, 161^3 126 / 103, 193^3 234 / 185; EPAIR
+// 97x120x120 54.8 / 58.6, 129^3 80.0 / 80.0, 50x300x200 107 / 115, 161^3 137 /
+// 129, 193^3 245 / 204.  The bit-exact and binary64 sweeps are bound by their
+// arithmetic and lose what the idle lanes cost (193^3 335 / 373)
+int z_width(const int nx, const long long cells)
+{
+    if (!kFast || cells < (kEPair ? 3LL << 20 : 1LL << 19)) return nx;
+    return (nx + 31) / 32 * 32;
+}
+static int z_width(const Geom& g) { return z_width(g.nx, (long long)g.nx * g.ny * g.nz); }
+
 // four-wave workgroups of one chunk of the x+y sweep over nz planes / of the
-// z sweep's flattened (x, y) columns
+// z sweep's flattened (x, y) columns, `width` of them a row
 static int xy_blocks(const Geom& g, const int nz)
 {
     const int waves = ((g.nx + 6) * nz + XY_TILE - 1) / XY_TILE;
     return (waves + 3) / 4;
 }
-static int z_blocks(const Geom& g) { return (g.nx * g.ny + 255) / 256; }
+static int z_blocks(const Geom& g, const int width) { return (width * g.ny + 255) / 256; }
 
 static int rows_grid(const Geom& g)
 {
@@ -1855,14 +1873,15 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
     } else if (dir == 1) {
         const int chunk = pick_chunk(g.ny, (int64_t)g.nx * nzr);
         dim3 grid((g.nx * nzr + 255) / 256, (g.ny + chunk - 1) / chunk);
-        hipLaunchKernelGGL((k_sweep_yz<1, MODE_ACC>), grid, dim3(256), 0, s, g, A, chunk);
+        hipLaunchKernelGGL((k_sweep_yz<1, MODE_ACC>), grid, dim3(256), 0, s, g, A, chunk, g.nx);
     } else {
-        const int nb = z_blocks(g);
+        const int width = z_width(g);
+        const int nb = z_blocks(g, width);
         const int chunk = std::min(z_march_limit(g), whole ? whole_march(nzr, nb, 2) : pick_chunk(nzr, (int64_t)g.nx * g.ny));
         const dim3 grid(nb, (nzr + chunk - 1) / chunk);
-        if (stage == 2)      hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE_NOR>), grid, dim3(256), 0, s, g, A, chunk);
-        else if (stage == 1) hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE>), grid, dim3(256), 0, s, g, A, chunk);
-        else                 hipLaunchKernelGGL((k_sweep_yz<2, MODE_CONV>), grid, dim3(256), 0, s, g, A, chunk);
+        if (stage == 2)      hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE_NOR>), grid, dim3(256), 0, s, g, A, chunk, width);
+        else if (stage == 1) hipLaunchKernelGGL((k_sweep_yz<2, MODE_STAGE>), grid, dim3(256), 0, s, g, A, chunk, width);
+        else                 hipLaunchKernelGGL((k_sweep_yz<2, MODE_CONV>), grid, dim3(256), 0, s, g, A, chunk, width);
     }
 }
 
@@ -1931,7 +1950,7 @@ void launch_test_face(const int n, const int dir, const void* stv, void* outv, h
 // the march length of a whole-block x+y (dir 3) or z (dir 2) launch that runs alone
 int whole_chunk(const Geom& g, const int dir)
 {
-    return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3) : whole_march(g.nz, z_blocks(g), 2);
+    return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3) : whole_march(g.nz, z_blocks(g, z_width(g)), 2);
 }
 
 // positions a wave of the fused x+y sweep stores
@@ -1944,10 +1963,11 @@ void xy_grid(const Geom& g, const int chunk, int dims[3])
     dims[0] = xy_blocks(g, g.nz); dims[1] = 1; dims[2] = (g.ny + chunk - 1) / chunk;
 }
 
-// grid of the z sweep: dims[0] blocks of 256 flattened (x, y) columns, dims[2] z-chunks
-void z_grid(const Geom& g, const int chunk, int dims[3])
+// grid of the z sweep: dims[0] blocks of 256 flattened (x, y) columns, `width` a
+// row, dims[2] z-chunks
+void z_grid(const Geom& g, const int width, const int chunk, int dims[3])
 {
-    dims[0] = z_blocks(g); dims[1] = 1; dims[2] = (g.nz + chunk - 1) / chunk;
+    dims[0] = z_blocks(g, width); dims[1] = 1; dims[2] = (g.nz + chunk - 1) / chunk;
 }
 
 void batch_sos(const BatchDev& B, const int blocks, const int cpu_form, const double cfl, const double dt_max,

@@ -40,6 +40,7 @@ struct CaseDesc
     double h;
     int bc[6];
     int chunk_xy, chunk_z; // march lengths of the x+y and z sweeps
+    int width_z;           // columns of a row of the z sweep (z_width)
     int nbx_xy, nby_xy;    // x+y sweep grid: x tiles, z groups (y chunks = third dim)
     int nbx_z, nby_z;      // z sweep grid: x blocks, y groups (z chunks = third dim)
     int nb_sos;            // speed-of-sound blocks
@@ -116,7 +117,8 @@ void persist_stage(const PersistDev& P, const int blocks[2], int threads, double
 int persist_occupancy(int threads, int phase);                                                             \
 int xy_tile();                                                                                             \
 void xy_grid(const Geom& g, int chunk, int dims[3]);                                                       \
-void z_grid(const Geom& g, int chunk, int dims[3]);                                                        \
+int z_width(int nx, long long cells);                                                                      \
+void z_grid(const Geom& g, int width, int chunk, int dims[3]);                                             \
 int whole_chunk(const Geom& g, int dir);                                                                   \
 } }
 

@@ -518,7 +518,7 @@ bool rebuild(mpcf_server* S)
                                : mpcf::detail::adaptive_march(c->g.ny, cols_xy);
         const int lz = n == 1 ? mpcf::fast::whole_chunk(c->g, 2)
                               : mpcf::detail::adaptive_march(c->g.nz, cols_z);
-        mpcf::detail::case_desc(c, c->cur, lxy, lz, hc[i], blocks);
+        mpcf::detail::case_desc(c, c->cur, lxy, lz, cells, hc[i], blocks);
         oxy[j + 1] = oxy[j] + blocks[0];
         oz[j + 1] = oz[j] + blocks[1];
         os[j + 1] = os[j] + blocks[2];
