@@ -11,6 +11,7 @@
 // PCIe until mpcf_download, and dt is produced and consumed on the device.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <condition_variable>
 #include <cstdio>
@@ -1137,15 +1138,22 @@ int batch_pull_cur(mpcf_batch* b)
 }
 
 // march length of case i in the x+y (which 0) or z sweep; `columns` is the
-// marching columns of all cases in that sweep
-int march_len(const mpcf_batch* b, int i, int nd, int which, long long columns)
+// marching columns of all cases in that sweep, `cells` their cells
+int march_len(const mpcf_batch* b, int i, int nd, int which, long long columns, long long cells)
 {
     const int forced = which == 0 ? b->chunk_xy[i] : b->chunk_z[i];
     const std::map<int, int>& tuned_map = which == 0 ? b->tuned_xy : b->tuned_z;
     auto it = tuned_map.find(nd);
     const int tuned = it != tuned_map.end() ? it->second : 0;
     if (forced > 0 || tuned > 0) return mpcf::detail::batch_march(nd, forced, tuned);
-    return mpcf::detail::adaptive_march(nd, columns);
+    // a queue item costs more than a block of a flat launch: the persistent
+    // launches keep marches of eight cells or more (16 cases of 32^3 220 us a
+    // step, 253 with the flat launches' 4)
+    if (b->mode == MPCF_BATCH_MODE_PERSISTENT) return mpcf::detail::adaptive_march(nd, columns, LLONG_MAX);
+    // a lone case marches as a single-case launch would (64^3 151 -> 115 us,
+    // bit-exact 128^3 1.13 -> 0.98 ms a step)
+    if (b->cases.size() == 1) return b->L->whole_chunk(b->cases[i]->g, which == 0 ? 3 : 2);
+    return mpcf::detail::adaptive_march(nd, columns, cells);
 }
 
 // the queues of the persistent stage launches: the x+y items of every case,
@@ -1241,8 +1249,8 @@ int batch_rebuild(mpcf_batch* b)
         int* oz = oxy + (b->cap + 1);
         int* os = oxy + 2 * (b->cap + 1);
         int blocks[3];
-        mpcf::detail::case_desc(c, c->cur, march_len(b, i, c->g.ny, 0, cols_xy), march_len(b, i, c->g.nz, 1, cols_z),
-                                cells, desc[i], blocks);
+        mpcf::detail::case_desc(c, c->cur, march_len(b, i, c->g.ny, 0, cols_xy, cells),
+                                march_len(b, i, c->g.nz, 1, cols_z, cells), cells, desc[i], blocks);
         oxy[j + 1] = oxy[j] + blocks[0];
         oz[j + 1] = oz[j] + blocks[1];
         os[j + 1] = os[j] + blocks[2];

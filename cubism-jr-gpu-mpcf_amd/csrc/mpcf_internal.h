@@ -73,6 +73,7 @@ struct Launchers
     decltype(&mpcf::parity::xy_tile) xy_tile;
     decltype(&mpcf::parity::xy_grid) xy_grid;
     decltype(&mpcf::parity::z_width) z_width;
+    decltype(&mpcf::parity::whole_chunk) whole_chunk;
 };
 
 #define MPCF_LAUNCHERS(NS)                                                                           \
@@ -83,7 +84,7 @@ struct Launchers
      mpcf::NS::launch_test_weno,                                                                      \
      mpcf::NS::launch_test_face,                                                                      \
      mpcf::NS::batch_sos, mpcf::NS::batch_xy, mpcf::NS::batch_z, mpcf::NS::persist_stage,        \
-     mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid, mpcf::NS::z_width}
+     mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid, mpcf::NS::z_width, mpcf::NS::whole_chunk}
 
 inline const Launchers kParity = MPCF_LAUNCHERS(parity);
 inline const Launchers kFast = MPCF_LAUNCHERS(fast);
@@ -286,20 +287,29 @@ inline bool has_halo(const int bc[6])
 // marched axis until the active cases together have about 2^17 marching
 // threads (two waves per SIMD), then round the length down to a power of two
 // between 8 and 64.  A step's latency is the march length times the per-cell
-// latency, so few small cases run short marches; long marches recompute fewer
-// warm-up cells.  Lengths that leave the grid just over a whole number of
-// resident rounds of blocks are slow, and powers of two avoid them for the
-// cubic sizes served here (measured on MI355X, one 192^3 case: 2.06 ms per
-// step with 64-cell marches, 2.16 with 32, 2.35 with 48, 2.83 with 96).
-// `columns` is the marching columns of all active cases in this sweep.
-inline int adaptive_march(const int nd, const long long columns)
+// latency; long marches recompute fewer warm-up cells.  Lengths that leave the
+// grid just over a whole number of resident rounds of blocks are slow, and
+// powers of two avoid them for the cubic sizes served here (measured on
+// MI355X, one 192^3 case: 2.06 ms per step with 64-cell marches, 2.16 with 32,
+// 2.35 with 48, 2.83 with 96).  Cases too few to give every such thread eight
+// cells all march the same 1, 2, 4 or 8 cells, whatever their extent: eight
+// left most of the chip idle (fast / bit-exact us a step, 8 cells and this
+// rule: 4 cases of 24^3..32^3 186 / 403 and 144 / 166, 16 of 32^3 217 / 506
+// and 182 / 360, 4 of 48^3 222 / 506 and 174 / 334; from 2^20 cells both equal).
+// `columns` is the marching columns of all active cases in this sweep, `cells`
+// their cells.
+inline int adaptive_march(const int nd, const long long columns, const long long cells)
 {
     const long long target = 1LL << 17;
-    long long nchunks = columns > 0 ? (target + columns - 1) / columns : 1;
-    if (nchunks < 1) nchunks = 1;
-    const int want = (int)((nd + nchunks - 1) / nchunks);
     int len = 8;
-    while (len * 2 <= want && len < 64) len *= 2;
+    if (cells < 8 * target) {
+        // the power of two nearest the cells a thread gets (up from 1.5 times)
+        for (len = 1; 3 * len * target <= 2 * cells; len *= 2) {}
+    } else {
+        const long long nchunks = columns > 0 ? (target + columns - 1) / columns : 1;
+        const int want = (int)((nd + nchunks - 1) / nchunks);
+        while (len * 2 <= want && len < 64) len *= 2;
+    }
     return len < nd ? len : nd;
 }
 

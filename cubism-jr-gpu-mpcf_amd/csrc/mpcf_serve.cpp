@@ -515,9 +515,9 @@ bool rebuild(mpcf_server* S)
         // (shorter chunks, more waves to fill the chip); a mix shares the
         // chip and takes the longer, cheaper chunks of adaptive_march
         const int lxy = n == 1 ? mpcf::fast::whole_chunk(c->g, 3)
-                               : mpcf::detail::adaptive_march(c->g.ny, cols_xy);
+                               : mpcf::detail::adaptive_march(c->g.ny, cols_xy, cells);
         const int lz = n == 1 ? mpcf::fast::whole_chunk(c->g, 2)
-                              : mpcf::detail::adaptive_march(c->g.nz, cols_z);
+                              : mpcf::detail::adaptive_march(c->g.nz, cols_z, cells);
         mpcf::detail::case_desc(c, c->cur, lxy, lz, cells, hc[i], blocks);
         oxy[j + 1] = oxy[j] + blocks[0];
         oz[j + 1] = oz[j] + blocks[1];
