@@ -1082,7 +1082,7 @@ struct mpcf_batch
     int cap = 0;
     bool dirty = true;
     bool cur_on_device = false;              // d_cur holds the truth (after steps)
-    // the cases in kBatchGroups groups of about equal cells, each stepped on
+    // the cases in up to kBatchGroups groups of about equal cells, each stepped on
     // its own stream (groups 1.. on side streams forked from and joined back
     // to `stream`), so that one group's x+y sweep runs beside another's z sweep
     int tot_xy[kBatchGroups] = {}, tot_z[kBatchGroups] = {}, tot_sos[kBatchGroups] = {};
@@ -1238,7 +1238,9 @@ int batch_rebuild(mpcf_batch* b)
     {
         std::vector<long long> cc(n);
         for (int i = 0; i < n; ++i) cells += cc[i] = (long long)b->cases[i]->g.nx * b->cases[i]->g.ny * b->cases[i]->g.nz;
-        split_groups(cc.data(), n, kBatchGroups, first);
+        const int groups = batch_groups(cells);
+        split_groups(cc.data(), n, groups, first);
+        for (int grp = groups; grp < kBatchGroups; ++grp) first[grp + 1] = n;   // the rest stay empty
     }
     for (int i = 0; i < n; ++i) {
         mpcf_ctx* c = b->cases[i];

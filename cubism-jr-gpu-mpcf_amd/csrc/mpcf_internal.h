@@ -93,10 +93,10 @@ inline const Launchers kFastPE = MPCF_LAUNCHERS(fastpe);
 inline const Launchers kF64 = MPCF_LAUNCHERS(f64);
 #undef MPCF_LAUNCHERS
 
-// batches and the server step their cases as this many groups of about equal
-// cells, each on its own stream (measured on a 64-case ensemble: four groups
-// serve a static batch best; the server, whose p99 under a request stream
-// suffers from more groups, uses two)
+// batches and the server step their cases as at most this many groups of about
+// equal cells, each on its own stream (measured on a 64-case ensemble: four
+// groups serve a static batch best; the server, whose p99 under a request
+// stream suffers from more groups, uses two)
 #ifndef MPCF_BATCH_GROUPS
 #define MPCF_BATCH_GROUPS 4
 #endif
@@ -123,6 +123,18 @@ inline void split_groups(const long long* cells, const int n, const int G, int* 
         first[g] = i;
     }
     first[G] = n;
+}
+
+// groups of a batch of `cells` cells: a stage's two launches are a few
+// microseconds each while the batch is small, and more groups only add launches
+// (us a step with 4, 2, 1 groups, fast build: 4 cases of 24^3..32^3 145, 83, 73;
+// 4 of 32^3 145, 93, 90; 16 of 32^3 183, 169, 174; 8 of 32^3..56^3 255, 256, 303;
+// 6 of 40^3..100^3 422, 411, 457, bit-exact 925, 1004, 1005; 24 of 32^3..96^3
+// 1588, 1628, 1915)
+inline int batch_groups(const long long cells)
+{
+    const int G = cells < (1LL << 17) ? 1 : cells < (1LL << 20) ? 2 : kBatchGroups;
+    return G < kBatchGroups ? G : kBatchGroups;
 }
 
 inline const unsigned kAllFlags = MPCF_FLAG_FAST | MPCF_FLAG_SOS_CPU | MPCF_FLAG_SPLIT_XY | MPCF_FLAG_FUSED_XY |
@@ -165,6 +177,7 @@ using mpcf::detail::pick_launchers;
 using mpcf::detail::kBatchGroups;
 using mpcf::detail::kServerGroups;
 using mpcf::detail::split_groups;
+using mpcf::detail::batch_groups;
 using mpcf::detail::elem_bytes;
 using mpcf::detail::kA;
 using mpcf::detail::kB;

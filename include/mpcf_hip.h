@@ -335,7 +335,7 @@ int mpcf_batch_set_march(mpcf_batch* batch, int case_id, int len_xy, int len_z);
  *     y-chunk) or z sweep (`threads` columns over one z-chunk) -- largest case
  *     first, until the queue is empty.  threads: workgroup size, 64, 128 or
  *     256 (0: 256).
- *   MPCF_BATCH_MODE_GROUPS (default): the cases in four groups of about equal
+ *   MPCF_BATCH_MODE_GROUPS (default): the cases in up to four groups of about equal
  *     cells, each on its own stream, with one flat launch per kernel kind per
  *     stage. */
 enum { MPCF_BATCH_MODE_GROUPS = 0, MPCF_BATCH_MODE_PERSISTENT = 1 };
