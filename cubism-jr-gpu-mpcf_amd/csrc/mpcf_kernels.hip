@@ -143,6 +143,34 @@ __device__ __forceinline__ SosIn take_folded(const StepState* st)
     return in;
 }
 
+struct DtArgs
+{
+    int with_dt;                  // 0: only the maximum (mpcf_max_sos)
+    double cfl, h, dt_max;
+};
+
+__device__ __forceinline__ void sos_finalize(StepState* st, const DtArgs& d, const SosIn& in)
+{
+    const double sos = in.sos;
+    st->sos_d = sos;
+    st->sos = (float)sos;
+    st->sos_is_d = kSosD ? 1 : 0;
+    st->bad = in.bad;
+    // the folded maximum (and flag) of the next step starts from zero
+    __hip_atomic_store(&st->next_sos_bits, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&st->next_sos_bits_d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&st->next_bad, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (d.with_dt) {
+        // binary64 dt from the binary32 (or binary64) maximum
+        double dt = d.cfl*d.h/sos;
+        dt = d.dt_max < dt ? d.dt_max : dt;
+        st->dt = dt;
+        st->h = d.h; st->cfl = d.cfl; st->dt_max = d.dt_max;
+        st->dtinvh = (float)(dt/d.h);
+        st->dtinvh_d = dt/d.h;
+    }
+}
+
 typedef FaceFluxT<Real> FaceFlux;
 typedef CellRecT<Real> CellRec;
 typedef RecT<Real> Rec;
@@ -1130,9 +1158,14 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
 #else
 #define MPCF_XY_WAVES
 #endif
-template <bool FIRST>
+// DT (a step's first stage, which needs no dt): one wave, of the tile that is
+// least often full, also turns the maximum that the previous step folded into
+// dt, for the z sweep that follows.  A launch of its own took 5 us with the gap
+// before it (16^3 40.3 -> 37.8 us a step, 64^3 93.5 -> 92.7, bit-exact 64^3
+// 201.4 -> 200.5; a step by itself 66 -> 52 us at 16^3)
+template <bool FIRST, bool DT>
 __global__ __launch_bounds__(256) MPCF_XY_WAVES
-void k_sweep_xy(const Geom g, const StageArgs A, const int chunk)
+void k_sweep_xy(const Geom g, const StageArgs A, const int chunk, StepState* dt_st, const DtArgs d)
 {
     // where a pipelined step's z sweep shares a SIMD with these waves, they
     // issue first (wave priority, not a queue priority): 512^3 19.92 ->
@@ -1140,6 +1173,9 @@ void k_sweep_xy(const Geom g, const StageArgs A, const int chunk)
     __builtin_amdgcn_s_setprio(2);
     const int gx = gridDim.x;
     const int t = xcd_order(blockIdx.x + blockIdx.y * gx, gx * gridDim.y);
+    if constexpr (DT) {
+        if (t == gx - 1 && threadIdx.y == 3 && threadIdx.x == 0) sos_finalize(dt_st, d, take_folded(dt_st));
+    }
     sweep_xy_body<FIRST, kSyncXY>(g, A, chunk, (t % gx) * 4 + threadIdx.y, threadIdx.y, t / gx);
 }
 
@@ -1231,12 +1267,6 @@ void k_halo(const Geom g, Real* __restrict__ u, const int64_t fs, const int face
 // the reduction target and the counter back to zero for the next step.
 // ---------------------------------------------------------------------------
 
-struct DtArgs
-{
-    int with_dt;                  // 0: only the maximum (mpcf_max_sos)
-    double cfl, h, dt_max;
-};
-
 // the finished reduction's targets, put back to zero with its counter
 __device__ __forceinline__ SosIn take_reduction(StepState* st)
 {
@@ -1246,28 +1276,6 @@ __device__ __forceinline__ SosIn take_reduction(StepState* st)
     in.bad = atomicExch(&st->bad_bits, 0u);
     atomicExch(&st->sos_count, 0u);
     return in;
-}
-
-__device__ __forceinline__ void sos_finalize(StepState* st, const DtArgs& d, const SosIn& in)
-{
-    const double sos = in.sos;
-    st->sos_d = sos;
-    st->sos = (float)sos;
-    st->sos_is_d = kSosD ? 1 : 0;
-    st->bad = in.bad;
-    // the folded maximum (and flag) of the next step starts from zero
-    __hip_atomic_store(&st->next_sos_bits, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&st->next_sos_bits_d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&st->next_bad, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (d.with_dt) {
-        // binary64 dt from the binary32 (or binary64) maximum
-        double dt = d.cfl*d.h/sos;
-        dt = d.dt_max < dt ? d.dt_max : dt;
-        st->dt = dt;
-        st->h = d.h; st->cfl = d.cfl; st->dt_max = d.dt_max;
-        st->dtinvh = (float)(dt/d.h);
-        st->dtinvh_d = dt/d.h;
-    }
 }
 
 // rows a wave of the reduction reads at a time
@@ -1863,8 +1871,12 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
         const int chunk = whole ? whole_march(g.ny, nb, 3) : pick_chunk(g.ny, (int64_t)g.nx * nzr);
         const dim3 grid(nb, (g.ny + chunk - 1) / chunk);
         // a first stage of a folded build does not read R
-        if (kFold && A.a == Real(0.0f)) hipLaunchKernelGGL(k_sweep_xy<true>, grid, dim3(64, 4), 0, s, g, A, chunk);
-        else                            hipLaunchKernelGGL(k_sweep_xy<false>, grid, dim3(64, 4), 0, s, g, A, chunk);
+        const bool first = kFold && A.a == Real(0.0f);
+        const DtArgs d{1, p.cfl, p.h, p.dt_max};
+        const dim3 block(64, 4);
+        if (p.dt_st) hipLaunchKernelGGL((k_sweep_xy<kFold, true>), grid, block, 0, s, g, A, chunk, p.dt_st, d);
+        else if (first) hipLaunchKernelGGL((k_sweep_xy<kFold, false>), grid, block, 0, s, g, A, chunk, p.dt_st, d);
+        else hipLaunchKernelGGL((k_sweep_xy<false, false>), grid, block, 0, s, g, A, chunk, p.dt_st, d);
     } else if (dir == 0) {
         const int npen = g.ny * nzr;
         const int chunk = pick_chunk(g.nx, npen);
