@@ -530,11 +530,11 @@ namespace {
 
 // pinned chunks of at least `want` bytes (at most kChunkMax), allocated; the
 // caller holds P.mu.  Small transfers get along with small chunks: pinning
-// 128 MB costs more than they do
+// 128 MB costs more than they do.  false: the host has no such memory left
 constexpr size_t kChunkMin = size_t(4) << 20, kChunkMax = size_t(64) << 20;
-int ready_chunks(PinnedChunks& P, const size_t want)
+bool ready_chunks(PinnedChunks& P, const size_t want)
 {
-    if (P.cap >= want) return MPCF_OK;
+    if (P.cap >= want) return true;
     const size_t cap = want <= kChunkMin ? kChunkMin : kChunkMax;
     char* b[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
@@ -545,14 +545,15 @@ int ready_chunks(PinnedChunks& P, const size_t want)
     if (e != hipSuccess) {
         for (int i = 0; i < 2; ++i)
             if (b[i]) hipHostFree(b[i]);
-        return fail(MPCF_EHIP, std::string("transfer staging: ") + hipGetErrorString(e));
+        (void)hipGetLastError();
+        return false;
     }
     for (int i = 0; i < 2; ++i) {
         if (P.buf[i]) hipHostFree(P.buf[i]);
         P.buf[i] = b[i];
     }
     P.cap = cap;
-    return MPCF_OK;
+    return true;
 }
 
 }  // namespace
@@ -569,7 +570,7 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
 {
     char* const dev = (char*)devv;
     const size_t n = (size_t)nh * per;
-    if (n < (size_t(1) << 18)) {
+    auto pageable = [&]() -> int {
         for (int q = 0; q < nh; ++q) {
             if (to_device) HIP_TRY(hipMemcpyAsync(dev + q * per, host[q], per, hipMemcpyHostToDevice, s));
             else {
@@ -578,13 +579,13 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
             }
         }
         return MPCF_OK;
-    }
+    };
+    if (n < (size_t(1) << 18)) return pageable();
     PinnedChunks& P = pinned_chunks();
     std::lock_guard<std::mutex> lk(P.mu);
     // at least four chunks, so that the two copies of most of them overlap
     const size_t cap = std::min(kChunkMax, std::max(size_t(1) << 20, (n / 4 + 4095) / 4096 * 4096));
-    const int rc = ready_chunks(P, cap);
-    if (rc != MPCF_OK) return rc;
+    if (!ready_chunks(P, cap)) return pageable();   // no pinned memory to be had
     const size_t nchunk = (n + cap - 1) / cap;
     auto length = [&](const size_t k) { return std::min(cap, n - k * cap); };
     // chunk k of the host arrays <-> its pinned buffer, by the pool of threads
