@@ -127,21 +127,21 @@ int pipeline_slabs(const mpcf_ctx* c)
 {
     if (c->pipe_req >= 0) return c->pipe_req;
     // the split sweeps are all VALU-bound: slabs give them nothing to overlap
-    // (measured on MI355X at 512^3, bit-exact build: whole-block 59.4 ms a
-    // step, 4 slabs 60.1, 8 slabs 61.4)
+    // (measured on MI355X at 512^3, bit-exact build: whole-block 50.3 ms a
+    // step, 4 slabs 50.5, 8 slabs 51.8)
     if (split_xy(c)) return 0;
     // so is the bit-exact binary32 build's fused sweep, whose division and
     // binary64 weight sequences make both sweeps VALU-bound (512^3: whole-
-    // block 57.05 ms a step, 4 slabs 57.6, 8 slabs 57.9; 384^3: whole 25.16,
-    // 3 slabs 25.17, 6 slabs 25.3)
+    // block 48.1 ms a step, 4 slabs 49.4, 8 slabs 49.9; 384^3: whole 20.2,
+    // 3 slabs 20.6, 6 slabs 21.0)
     if (!(c->flags & MPCF_FLAG_FAST)) return 0;
     // blocks of 2^24 cells or more, slabs by depth as measured on MI355X (fast
-    // build, cubes, ms a step): 256^3 4 slabs (2.66; 2.74 with 2, 2.81
-    // whole); 320^3 3 (4.83; 4.97 with 4, 4.98 with 5); 384^3 3 (8.29; 8.34
-    // with 4, 8.49 with 6); 448^3 4 (13.0; 13.2 with 7); 512^3 8 (19.8;
-    // 20.0-20.1 with 6 or 10, 20.3 with 12); 640^3 8 (10 slabs 3 % faster on
-    // one box, equal on another); 768^3 and 1024^3 8 (12 slabs were 6 %
-    // slower at 1024^3).  128^3 runs best whole.
+    // build, cubes, ms a step): 256^3 4 slabs (2.53; 2.62 with 2, 2.56
+    // whole); 320^3 3 (4.59; 4.73 with 4, 5.01 whole); 384^3 3 (7.87; 7.92
+    // with 4, 8.04 with 6); 448^3 4 (12.4; 12.6 with 7); 512^3 8 (18.7; 20.2
+    // with 6 or whole, 19.1 with 10, 19.2 with 12); 640^3 8 (10 slabs 3 %
+    // faster); 768^3 and 1024^3 8 (12 slabs 1 % faster at 768^3, 6 % slower at
+    // 1024^3).  128^3 runs best whole.
     const int64_t cells = (int64_t)c->g.nx * c->g.ny * c->g.nz;
     const int nz = c->g.nz;
     const int S = nz < 320 ? nz / 64 : nz < 512 ? nz / 100 : std::min(8, nz / 64);
