@@ -122,8 +122,9 @@ void run_rhs(mpcf_ctx* c, const void* u, void* uo, double a, double b, double dt
 }
 
 // z-slabs of a pipelined step (0: none): the count mpcf_set_pipeline asked
-// for, else one from the block's size
-int pipeline_slabs(const mpcf_ctx* c)
+// for, else one from the block's size.  queued: the step is one of several of
+// a call, whose slabs overlap from step to step
+int pipeline_slabs(const mpcf_ctx* c, const bool queued)
 {
     if (c->pipe_req >= 0) return c->pipe_req;
     // the split sweeps are all VALU-bound: slabs give them nothing to overlap
@@ -136,14 +137,22 @@ int pipeline_slabs(const mpcf_ctx* c)
     // 3 slabs 20.6, 6 slabs 21.0)
     if (!(c->flags & MPCF_FLAG_FAST)) return 0;
     // blocks of 2^24 cells or more, slabs by depth as measured on MI355X (fast
-    // build, cubes, ms a step): 256^3 4 slabs (2.53; 2.62 with 2, 2.56
-    // whole); 320^3 3 (4.59; 4.73 with 4, 5.01 whole); 384^3 3 (7.87; 7.92
-    // with 4, 8.04 with 6); 448^3 4 (12.4; 12.6 with 7); 512^3 8 (18.7; 20.2
-    // with 6 or whole, 19.1 with 10, 19.2 with 12); 640^3 8 (10 slabs 3 %
+    // build, cubes, ms a step): 320^3 3 slabs (4.49; 4.55 with 4, 4.96 whole);
+    // 384^3 3 (7.77; 7.82 with 4, 8.37 whole); 448^3 4 (12.24; 13.34 whole);
+    // 512^3 8 (18.5; 20.0 with 3 or whole, 19.1 with 10); 640^3 8 (10 slabs 3 %
     // faster); 768^3 and 1024^3 8 (12 slabs 1 % faster at 768^3, 6 % slower at
-    // 1024^3).  128^3 runs best whole.
+    // 1024^3)
     const int64_t cells = (int64_t)c->g.nx * c->g.ny * c->g.nz;
     const int nz = c->g.nz;
+    // up to 2^25 cells three slabs, in queued steps from 3 * 2^21 cells (a step
+    // by itself has no neighbour to overlap its ends, and from 2^24 as above),
+    // where a slab still has some 16 planes.  Whole / 3 slabs, us a step:
+    // 144^3 539 / 522 but 160^3 665 / 763, 192^3 1089 / 1004, (240,208,184) 1474 /
+    // 1417, (227,270,156) 1674 / 1504, 240^3 2238 / 1992, (400,400,60) 1507 / 1404,
+    // but (1000,1000,10) 1581 / 1770; a step by itself 192^3 1128 / 1116,
+    // (240,208,184) 1524 / 1565.  E as a pair between -9 and +7 %: not taken
+    if (!(c->flags & MPCF_FLAG_P64) && cells < (int64_t(1) << 25) && nz >= 48)
+        return (queued ? cells >= (int64_t(3) << 21) : cells >= (int64_t(1) << 24) && nz >= 128) ? 3 : 0;
     const int S = nz < 320 ? nz / 64 : nz < 512 ? nz / 100 : std::min(8, nz / 64);
     return (cells >= (int64_t(1) << 24) && S >= 2) ? S : 0;
 }
@@ -817,11 +826,12 @@ int step_args(mpcf_ctx* c, const double cfl, const double dt_max, const char* wh
 
 // one LSRK3 step, queued.  keep_open: a pipelined FAST step may leave its
 // last z sweeps unjoined (c->pipe_open) so that the next step's first x+y
-// sweeps overlap them; the caller joins before it returns.
-int step_queue(mpcf_ctx* c, const double cfl, const double dt_max, const bool keep_open)
+// sweeps overlap them; the caller joins before it returns.  queued: one of
+// several steps of the call.
+int step_queue(mpcf_ctx* c, const double cfl, const double dt_max, const bool keep_open, const bool queued)
 {
     // the sweeps apply the boundary conditions as they load: no ghost fill
-    const int slabs = pipeline_slabs(c);
+    const int slabs = pipeline_slabs(c, queued);
     // pipelined FAST steps run dt on the second stream, ahead of the first
     // stage's z sweeps, while the first stage's x+y sweeps (which need no dt)
     // start on the context's stream as soon as their slab of the previous
@@ -884,7 +894,7 @@ extern "C" int mpcf_step(mpcf_ctx* c, double cfl, double dt_max, double* dt)
 {
     int rc = step_args(c, cfl, dt_max, "mpcf_step");
     if (rc != MPCF_OK) return rc;
-    rc = step_queue(c, cfl, dt_max, false);
+    rc = step_queue(c, cfl, dt_max, false, false);
     if (rc != MPCF_OK) return rc;
     if (dt) {
         double d = 0;
@@ -903,8 +913,12 @@ extern "C" int mpcf_steps(mpcf_ctx* c, int nsteps, double cfl, double dt_max)
     int rc = step_args(c, cfl, dt_max, "mpcf_steps");
     if (rc != MPCF_OK) return rc;
     if (nsteps < 0) return fail(MPCF_EINVAL, "mpcf_steps: nsteps must be >= 0");
+    // a stream under capture keeps to the slabs of a step by itself
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(c->stream, &capturing));
+    const bool queued = nsteps > 1 && capturing == hipStreamCaptureStatusNone;
     for (int k = 0; k < nsteps; ++k) {
-        rc = step_queue(c, cfl, dt_max, k + 1 < nsteps);
+        rc = step_queue(c, cfl, dt_max, k + 1 < nsteps, queued);
         if (rc != MPCF_OK) {
             join_pipeline(c);
             return rc;
