@@ -122,9 +122,8 @@ void run_rhs(mpcf_ctx* c, const void* u, void* uo, double a, double b, double dt
 }
 
 // z-slabs of a pipelined step (0: none): the count mpcf_set_pipeline asked
-// for, else one from the block's size.  queued: the step is one of several of
-// a call, whose slabs overlap from step to step
-int pipeline_slabs(const mpcf_ctx* c, const bool queued)
+// for, else one from the block's size
+int pipeline_slabs(const mpcf_ctx* c)
 {
     if (c->pipe_req >= 0) return c->pipe_req;
     // the split sweeps are all VALU-bound: slabs give them nothing to overlap
@@ -137,24 +136,32 @@ int pipeline_slabs(const mpcf_ctx* c, const bool queued)
     // 3 slabs 20.6, 6 slabs 21.0)
     if (!(c->flags & MPCF_FLAG_FAST)) return 0;
     // blocks of 2^24 cells or more, slabs by depth as measured on MI355X (fast
-    // build, cubes, ms a step): 320^3 3 slabs (4.49; 4.55 with 4, 4.96 whole);
-    // 384^3 3 (7.77; 7.82 with 4, 8.37 whole); 448^3 4 (12.24; 13.34 whole);
-    // 512^3 8 (18.5; 20.0 with 3 or whole, 19.1 with 10); 640^3 8 (10 slabs 3 %
-    // faster); 768^3 and 1024^3 8 (12 slabs 1 % faster at 768^3, 6 % slower at
-    // 1024^3)
+    // build, cubes, ms a step): 256^3 4 slabs (2.50; 2.56 with 3, 2.55 whole);
+    // 320^3 3 (4.53; 4.68 with 4, 4.95 whole); 384^3 3 (7.77; 7.82 with 4,
+    // 8.37 whole); 448^3 4 (12.24; 13.34 whole); 512^3 8 (18.5; 20.0 with 3 or
+    // whole, 19.1 with 10); 640^3 8 (10 slabs 3 % faster); 768^3 and 1024^3 8
+    // (12 slabs 1 % faster at 768^3, 6 % slower at 1024^3)
     const int64_t cells = (int64_t)c->g.nx * c->g.ny * c->g.nz;
     const int nz = c->g.nz;
-    // up to 2^25 cells three slabs, in queued steps from 3 * 2^21 cells (a step
-    // by itself has no neighbour to overlap its ends, and from 2^24 as above),
-    // where a slab still has some 16 planes.  Whole / 3 slabs, us a step:
-    // 144^3 539 / 522 but 160^3 665 / 763, 192^3 1089 / 1004, (240,208,184) 1474 /
-    // 1417, (227,270,156) 1674 / 1504, 240^3 2238 / 1992, (400,400,60) 1507 / 1404,
-    // but (1000,1000,10) 1581 / 1770; a step by itself 192^3 1128 / 1116,
-    // (240,208,184) 1524 / 1565.  E as a pair between -9 and +7 %: not taken
-    if (!(c->flags & MPCF_FLAG_P64) && cells < (int64_t(1) << 25) && nz >= 48)
-        return (queued ? cells >= (int64_t(3) << 21) : cells >= (int64_t(1) << 24) && nz >= 128) ? 3 : 0;
     const int S = nz < 320 ? nz / 64 : nz < 512 ? nz / 100 : std::min(8, nz / 64);
     return (cells >= (int64_t(1) << 24) && S >= 2) ? S : 0;
+}
+
+// whether a step that is one of several of a call, whose slabs overlap from step
+// to step, takes three slabs with marches fitted to the chip (SweepParams::fit).
+// Not in a step by itself, whose ends have nothing to overlap, and only where a
+// slab has some 16 planes.  us a step, 3 such slabs against the whole block
+// below 2^24 cells and pipeline_slabs' count above: 144^3 522 / 539 but 160^3
+// 763 / 665, 192^3 1004 / 1089, (240,208,184) 1417 / 1474, (227,270,156) 1504 /
+// 1674, 240^3 1992 / 2238, (400,400,60) 1404 / 1507 but (1000,1000,10) 1770 /
+// 1581, 256^3 2323 / 2502, 320^3 4486 / 4526, 384^3 7803 / 7773; one step a
+// call 192^3 1116 / 1128, (240,208,184) 1565 / 1524.  E as a pair between -9
+// and +7 %: not taken
+bool fitted_slabs(const mpcf_ctx* c)
+{
+    const int64_t cells = (int64_t)c->g.nx * c->g.ny * c->g.nz;
+    return c->pipe_req < 0 && !split_xy(c) && (c->flags & MPCF_FLAG_FAST) && !(c->flags & MPCF_FLAG_P64) &&
+           cells >= (int64_t(3) << 21) && cells < (int64_t(1) << 25) && c->g.nz >= 48;
 }
 
 // the x+y sweeps of a step's first stage need no dt (the FAST builds store
@@ -177,8 +184,9 @@ bool dt_deferred(const mpcf_ctx* c)
 // the first stage's x+y sweep of slab j waits for that step's last z sweep of
 // slab j (which wrote the slab's u) instead of the whole step.  open: leave
 // this step open the same way (the caller's stream has not joined it).
-// skipR: the last stage's z sweeps do not store R.
-int run_stages_pipelined(mpcf_ctx* c, const int S, const bool prev_open, const bool open, const bool skipR)
+// skipR: the last stage's z sweeps do not store R.  fit: see fitted_slabs.
+int run_stages_pipelined(mpcf_ctx* c, const int S, const bool prev_open, const bool open, const bool skipR,
+                         const bool fit)
 {
     if (!c->stream2) HIP_TRY(hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
     while (c->pipe_ev.size() < (size_t)(2 * 3 * S)) {
@@ -195,6 +203,7 @@ int run_stages_pipelined(mpcf_ctx* c, const int S, const bool prev_open, const b
         p.a = kA[s]; p.b = kB[s]; p.dtinvh = 0.0; p.st = c->st;
         p.sos_next = s == 2 ? c->st : nullptr; p.sos_cpu = (c->flags & MPCF_FLAG_SOS_CPU) ? 1 : 0;
         p.bcmask = mpcf::detail::bc_mask(c->bc);
+        p.fit = fit;
         for (int j = 0; j < S; ++j) {
             p.z0 = (int)((int64_t)c->g.nz * j / S);
             p.z1 = (int)((int64_t)c->g.nz * (j + 1) / S);
@@ -831,7 +840,8 @@ int step_args(mpcf_ctx* c, const double cfl, const double dt_max, const char* wh
 int step_queue(mpcf_ctx* c, const double cfl, const double dt_max, const bool keep_open, const bool queued)
 {
     // the sweeps apply the boundary conditions as they load: no ghost fill
-    const int slabs = pipeline_slabs(c, queued);
+    const bool fit = queued && fitted_slabs(c);
+    const int slabs = fit ? 3 : pipeline_slabs(c);
     // pipelined FAST steps run dt on the second stream, ahead of the first
     // stage's z sweeps, while the first stage's x+y sweeps (which need no dt)
     // start on the context's stream as soon as their slab of the previous
@@ -872,7 +882,7 @@ int step_queue(mpcf_ctx* c, const double cfl, const double dt_max, const bool ke
     // R in its last stage: the next step's first stage multiplies it by a = 0
     const bool skipR = keep_open && dt_deferred(c);
     if (slabs) {
-        const int rc = run_stages_pipelined(c, slabs, prev_open, defer && keep_open, skipR);
+        const int rc = run_stages_pipelined(c, slabs, prev_open, defer && keep_open, skipR, fit);
         if (rc != MPCF_OK) return rc;
     } else {
         mpcf::SweepParams dt;

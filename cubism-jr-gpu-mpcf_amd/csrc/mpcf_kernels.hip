@@ -1764,18 +1764,19 @@ static int whole_march(const int nd, const int64_t blocks, const int dir)
     return best;
 }
 
-// March length of a FAST slab's fused x+y (dir 3) or z (dir 2) sweep in a block
-// of less than 2^25 cells, where a slab's launch is only a few workgroups a CU
-// and runs beside the other sweep's: the least rows on the busiest of the 256
-// CUs, as in whole_march, with at most five workgroups a CU -- longer marches
-// than pick_chunk's have fewer start-up rows, and counts just over a multiple
-// of 256 cost a round.  The x+y sweep keeps two workgroups a CU (a lone wave's
-// instructions do not pair: a slab of (216, 189, 62) in one workgroup a CU
+// March length of a FAST slab's fused x+y (dir 3) or z (dir 2) sweep where the
+// slab's launch is only a few workgroups a CU and runs beside the other sweep's
+// (SweepParams::fit: queued steps of blocks below 2^25 cells): the least rows on
+// the busiest of the 256 CUs, as in whole_march, with at most five workgroups a
+// CU -- longer marches than pick_chunk's have fewer start-up rows, and counts
+// just over a multiple of 256 cost a round.  The x+y sweep keeps two workgroups
+// a CU (a lone wave's instructions do not pair: slabs of (216, 189, 62) with one
 // takes 1.6 times as long a step).  Three slabs, FAST, ms a step, pick_chunk / this:
 // (216,189,186) 1.20 / 1.15, (227,270,156) 1.56 / 1.50, 240^3 2.15 / 1.99,
-// (221,248,290) 2.59 / 2.30, (270,235,266) 2.57 / 2.53, 256^3 2.56 / 2.32 (four
-// slabs 2.50 / 2.27), 320^3 4.53 / 4.49.  Larger blocks keep pick_chunk: 384^3
-// 7.77 / 7.80, 448^3 12.24 / 12.40.
+// (221,248,290) 2.59 / 2.30, (270,235,266) 2.57 / 2.53, 256^3 2.56 / 2.32,
+// 320^3 4.53 / 4.49.  Larger blocks keep pick_chunk: 384^3 7.77 / 7.80, 448^3
+// 12.24 / 12.40; so do other slab counts, which it suits less evenly (four slabs,
+// 256^3 2.50 / 2.27, (270,235,266) 2.64 / 2.87).
 static int slab_march(const int nd, const int64_t blocks, const int dir)
 {
     const double ov = dir == 3 ? 1.0 : 3.0;
@@ -1794,10 +1795,6 @@ static int slab_march(const int nd, const int64_t blocks, const int dir)
     }
     return best;
 }
-// whether a slab of block g marches by it (E as a pair and the binary64 steps
-// were not measured to gain and keep pick_chunk)
-static bool small_slabs(const Geom& g) { return kFast && !kP64 && (int64_t)g.nx * g.ny * g.nz < (int64_t(1) << 25); }
-
 // columns of a z sweep's rows of nx, in a launch (or a batch's launches) over
 // `cells` cells.  The FAST builds' z sweep runs at the memory's rate: rows
 // rounded up to 32 columns give every half wave one whole 128-byte line a
@@ -1902,7 +1899,7 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
     const bool whole = A.z0 == 0 && A.z1 == g.nz;   // not a slab
     if (dir == 3) {
         const int nb = xy_blocks(g, nzr);
-        const int chunk = whole ? whole_march(g.ny, nb, 3) : small_slabs(g) ? slab_march(g.ny, nb, 3)
+        const int chunk = whole ? whole_march(g.ny, nb, 3) : p.fit ? slab_march(g.ny, nb, 3)
                                                                             : pick_chunk(g.ny, (int64_t)g.nx * nzr);
         const dim3 grid(nb, (g.ny + chunk - 1) / chunk);
         // a first stage of a folded build does not read R
@@ -1924,7 +1921,7 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
     } else {
         const int width = z_width(g);
         const int nb = z_blocks(g, width);
-        const int march = whole ? whole_march(nzr, nb, 2) : small_slabs(g) ? slab_march(nzr, nb, 2)
+        const int march = whole ? whole_march(nzr, nb, 2) : p.fit ? slab_march(nzr, nb, 2)
                                                                            : pick_chunk(nzr, (int64_t)g.nx * g.ny);
         const int chunk = std::min(z_march_limit(g), march);
         const dim3 grid(nb, (nzr + chunk - 1) / chunk);

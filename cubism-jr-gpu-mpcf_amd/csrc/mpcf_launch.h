@@ -27,6 +27,7 @@ struct SweepParams
     double cfl = 0, h = 0, dt_max = 0;   // its arguments
     int z0 = 0, z1 = -1;            // z range of the fused x+y sweep's planes and the z sweep's
                                     // rows (a slab of a pipelined step); z1 < 0: the whole block
+    bool fit = false;               // a slab's march lengths fill whole rounds of the chip (slab_march)
     int bcmask;            // bit f: face f reflecting; bit 8+f: face f a halo face
                            // (ghost band imported); else absorbing.  The sweeps
                            // apply the boundary conditions as they load

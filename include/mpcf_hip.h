@@ -103,9 +103,9 @@ int mpcf_destroy(mpcf_ctx* ctx);
  * MPCF_FLAG_NO_PIPELINE): in the FAST builds, for blocks of 2^24 cells or
  * more, NZ/64 slabs for NZ < 320, NZ/100 for NZ < 512 and min(8, NZ/64)
  * above (the fastest counts measured on cubes), whole-block when that is
- * below 2 or the block is smaller; without P64 / E_PAIR, 3 slabs below 2^25
- * cells, in the steps of an mpcf_steps call (two or more, not under capture)
- * from 3 * 2^21 cells if NZ >= 48; in the bit-exact and binary64 builds and
+ * below 2 or the block is smaller; without P64 / E_PAIR, the steps of an
+ * mpcf_steps call (two or more, not under capture) take 3 slabs from 3 * 2^21
+ * to 2^25 cells if NZ >= 48; in the bit-exact and binary64 builds and
  * with the split sweeps, whole-block (their sweeps are all VALU-bound).  slabs <= min(64, NZ).  No counterpart in the
  * reference, whose stages run chunk by chunk on the host (GPUlab.cpp:703-793). */
 int mpcf_set_pipeline(mpcf_ctx* ctx, int slabs);

@@ -1,8 +1,9 @@
 """Which FAST blocks step in z-slabs on their own, and how far a slab's sweeps
 march.  Slabs and march lengths decide which launch computes a cell, never its
-value: either side of the rule's lines (6.3 M and 16.8 M cells, 48 planes), with ragged
-slabs, and in forced slabs whose launches are too few for the chip, steps equal
-the whole block's bit for bit, queued and one a call."""
+value: either side of the rule's lines (6.3 M cells, 48 planes, 2^24 cells for
+a step by itself), with ragged slabs, and in forced slabs whose launches are too
+few for the chip, steps equal the whole block's bit for bit, queued and one a
+call."""
 import numpy as np
 import pytest
 
