@@ -852,6 +852,16 @@ __device__ __forceinline__ Real from_right(const Real edge, const Real v) { retu
 // lane 63 (kHaloLDS)
 typedef Real Halo4 __attribute__((ext_vector_type(4)));
 
+// orders the wave's LDS accesses before it against those after it, for all its
+// lanes: LDS serves one wave's accesses in order, so it holds the compiler back
+// and costs no instruction
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ Prim prim_from_left(const Prim& q)
 {
     Prim o;
@@ -1037,10 +1047,13 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
         if (xmirror) o[FU] *= sgx;
     };
 
-    __shared__ Halo4 sh_halo[kHaloLDS ? 4 : 1][kHaloLDS ? kHaloRows : 1][NVAR];
+    // scalars, a Halo4 each: four lanes write the four positions of one, and a
+    // store into an element of a vector reads and writes the whole vector
+    __shared__ alignas(sizeof(Halo4)) Real sh_halo[kHaloLDS ? 4 : 1][kHaloLDS ? kHaloRows : 1][NVAR][4];
     // primitives beside the wave of rows [h0, h0 + kHaloRows), interior rows
     int h0 = c0 - kHaloRows;
     auto fill_halo = [&](const int row0) {
+        wave_sync();   // the wave's lanes have read the rows that go
         h0 = row0;
         const int j = lane >> 2, side = lane & 3;
         const int row = min(row0 + j, c1 - 1);
@@ -1058,9 +1071,8 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
         const Prim p = prim_of(w);
         const Real v[NVAR] = {p.r, p.u, p.v, p.w, p.p, p.G, p.P};
 #pragma unroll
-        for (int f = 0; f < NVAR; ++f) {
-            sh_halo[wib][j][f][side] = v[f];
-        }
+        for (int f = 0; f < NVAR; ++f) sh_halo[wib][j][f][side] = v[f];
+        wave_sync();   // the rows are there for every lane
     };
 
     March<1, MODE_ACC> m;
@@ -1100,7 +1112,7 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
                 Halo4 halo[NVAR];
 #pragma unroll
                 for (int f = 0; f < NVAR; ++f)
-                    if constexpr (kHaloLDS) halo[f] = sh_halo[wib][k - 1 - h0][f];
+                    if constexpr (kHaloLDS) halo[f] = *(const Halo4*)sh_halo[wib][k - 1 - h0][f];
                 const CellRec rx = reconstruct_lanes<SYNC>(m.w1, halo);
                 const Prim Lm = prim_from_left(rx.m);
                 const FaceFlux Fxl = riemann<0, Real, kFast, SYNC>(Lm, rx.p);      // face x-1/2
