@@ -1089,6 +1089,22 @@ extern "C" int mpcf_test_face(int n, int dir, const float* st, float* out, unsig
     return MPCF_OK;
 }
 
+extern "C" int mpcf_test_rows(int n, const float* st, int* again, unsigned flags)
+{
+    if (n < 0 || (n > 0 && (!st || !again))) return fail(MPCF_EINVAL, "mpcf_test_rows: bad argument");
+    if (n == 0) return MPCF_OK;
+    if (flags & MPCF_FLAG_FP64) return fail(MPCF_EINVAL, "mpcf_test_rows: binary32 arrays only");
+    const Launchers* L = pick_launchers(flags);
+    DevBuf a, o;
+    HIP_TRY(hipMalloc(&a.p, sizeof(float) * 7 * 68 * (size_t)n));
+    HIP_TRY(hipMalloc(&o.p, sizeof(int) * (size_t)n));
+    HIP_TRY(hipMemcpy(a.p, st, sizeof(float) * 7 * 68 * (size_t)n, hipMemcpyHostToDevice));
+    L->test_rows(n, a.p, (int*)o.p, nullptr);
+    LAUNCH_CHECK("test_rows");
+    HIP_TRY(hipMemcpy(again, o.p, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost));
+    return MPCF_OK;
+}
+
 // ===========================================================================
 // Batched ensembles (mpcf_batch_*): many independent cases of uneven sizes
 // advanced together, one launch per kernel kind per stage, per-case dt on the

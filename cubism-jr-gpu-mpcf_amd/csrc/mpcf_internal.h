@@ -65,6 +65,7 @@ struct Launchers
     decltype(&mpcf::parity::launch_stream) stream;
     decltype(&mpcf::parity::launch_test_weno) test_weno;
     decltype(&mpcf::parity::launch_test_face) test_face;
+    decltype(&mpcf::parity::launch_test_rows) test_rows;
     decltype(&mpcf::parity::batch_sos) b_sos;
     decltype(&mpcf::parity::batch_xy) b_xy;
     decltype(&mpcf::parity::batch_z) b_z;
@@ -82,7 +83,7 @@ struct Launchers
      mpcf::NS::launch_sweep, mpcf::NS::launch_update,                                                            \
      mpcf::NS::launch_pack, mpcf::NS::launch_pack_epair, mpcf::NS::launch_stream,                      \
      mpcf::NS::launch_test_weno,                                                                      \
-     mpcf::NS::launch_test_face,                                                                      \
+     mpcf::NS::launch_test_face, mpcf::NS::launch_test_rows,                                          \
      mpcf::NS::batch_sos, mpcf::NS::batch_xy, mpcf::NS::batch_z, mpcf::NS::persist_stage,        \
      mpcf::NS::persist_occupancy, mpcf::NS::xy_tile, mpcf::NS::xy_grid, mpcf::NS::z_width, mpcf::NS::whole_chunk}
 

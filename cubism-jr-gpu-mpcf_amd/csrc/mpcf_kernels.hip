@@ -862,6 +862,12 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The x faces of a wave, each lane's face to its left: lane 0 has no left state
+// (it reads zeros), and its face is not used.  Counted among the faces whose
+// operands decide on the quick quotients, it had every wave solve every x face
+// of the bit-exact build twice
+constexpr uint64_t kXFaceLanes = ~uint64_t(1);
+
 __device__ __forceinline__ Prim prim_from_left(const Prim& q)
 {
     Prim o;
@@ -927,11 +933,12 @@ __device__ __forceinline__ CellRec reconstruct_lanes_as(const Prim& c, const Hal
 // as reconstruct(): the bit-exact builds take the quick quotients, and the
 // IEEE ones where a lane's window needs them
 template <bool SYNC>
-__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c, const Halo4* halo)
+__device__ __forceinline__ CellRec reconstruct_lanes(const Prim& c, const Halo4* halo, bool* again = nullptr)
 {
     if constexpr (!kFast) {
         bool odd = false;
         CellRec o = reconstruct_lanes_as<SYNC, true>(c, halo, &odd);
+        if (again) *again = any_lane(odd);
         if (__builtin_expect(any_lane(odd), 0)) o = reconstruct_lanes_as<SYNC, false>(c, halo, nullptr);
         return o;
     } else {
@@ -1115,7 +1122,7 @@ __device__ __forceinline__ void sweep_xy_body(const Geom& g, const StageArgs& A,
                     if constexpr (kHaloLDS) halo[f] = *(const Halo4*)sh_halo[wib][k - 1 - h0][f];
                 const CellRec rx = reconstruct_lanes<SYNC>(m.w1, halo);
                 const Prim Lm = prim_from_left(rx.m);
-                const FaceFlux Fxl = riemann<0, Real, kFast, SYNC>(Lm, rx.p);      // face x-1/2
+                const FaceFlux Fxl = riemann<0, Real, kFast, SYNC, kXFaceLanes>(Lm, rx.p);      // face x-1/2
                 FaceFlux Fxr;                                                        // face x+1/2
 #pragma unroll
                 for (int f = 0; f < NVAR; ++f) Fxr.f[f] = from_right(Fxl.f[f]);
@@ -1536,6 +1543,35 @@ __global__ void k_test_face(const int n, const Real* __restrict__ st, Real* __re
     Real* o = out + 12*(int64_t)i;
     for (int q = 0; q < NVAR; ++q) o[q] = F.f[q];
     o[7] = F.vel; o[8] = left.m.G; o[9] = right.p.G; o[10] = left.m.P; o[11] = right.p.P;
+}
+
+// st: n rows x 7 fields x 68 cells, conserved; row i is what a wave of the x+y
+// sweep holds in x (its 64 lanes' cells and two beside them on either side).
+// again[i]: bit 0, the wave evaluated its windows, bit 1, its faces a second
+// time with the IEEE quotients
+__global__ void k_test_rows(const Real* __restrict__ st, int* __restrict__ again)
+{
+    const int lane = threadIdx.x;
+    const Real* const s = st + (int64_t)blockIdx.x * NVAR * 68;
+    auto prim = [&](const int cell) {
+        Real w[NU] = {};
+#pragma unroll
+        for (int f = 0; f < NVAR; ++f) w[f] = s[f * 68 + cell];
+        return prim_of(w);
+    };
+    Halo4 halo[NVAR];
+#pragma unroll
+    for (int side = 0; side < 4; ++side) {
+        const Prim p = prim(side < 2 ? side : 64 + side);
+        const Real v[NVAR] = {p.r, p.u, p.v, p.w, p.p, p.G, p.P};
+#pragma unroll
+        for (int f = 0; f < NVAR; ++f) halo[f][side] = v[f];
+    }
+    bool windows = false, faces = false;
+    const CellRec rx = reconstruct_lanes<false>(prim(2 + lane), halo, &windows);
+    const Prim Lm = prim_from_left(rx.m);
+    (void)riemann<0, Real, kFast, false, kXFaceLanes>(Lm, rx.p, &faces);
+    if (lane == 0) again[blockIdx.x] = (windows ? 1 : 0) | (faces ? 2 : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1993,6 +2029,11 @@ void launch_test_weno(const int n, const void* in5v, void* mv, void* pv, hipStre
     Real* m = (Real*)mv;
     Real* p = (Real*)pv;
     hipLaunchKernelGGL(k_test_weno, dim3((n + 255) / 256), dim3(256), 0, s, n, in5, m, p);
+}
+
+void launch_test_rows(const int n, const void* st, int* again, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_test_rows, dim3(n), dim3(64), 0, s, (const Real*)st, again);
 }
 
 void launch_test_face(const int n, const int dir, const void* stv, void* outv, hipStream_t s)

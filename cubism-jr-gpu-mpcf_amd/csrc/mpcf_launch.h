@@ -112,6 +112,7 @@ void launch_pack_epair(const Geom& g, void* hi, void* lo, void* dense, int to_pa
 void launch_stream(const Geom& g, void* pad, float* dense, int kind, int out, hipStream_t s);             \
 void launch_test_weno(int n, const void* in5, void* m, void* p, hipStream_t s);                            \
 void launch_test_face(int n, int dir, const void* st, void* out, hipStream_t s);                           \
+void launch_test_rows(int n, const void* st, int* again, hipStream_t s);                                   \
 void batch_sos(const BatchDev& B, int blocks, int cpu_form, double cfl, double dt_max, hipStream_t s);    \
 void batch_xy(const BatchDev& B, int blocks, double a, double b, hipStream_t s);                           \
 void batch_z(const BatchDev& B, int blocks, double a, double b, int fold, int cpu_form, int storeR,         \

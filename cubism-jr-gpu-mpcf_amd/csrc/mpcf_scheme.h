@@ -156,14 +156,14 @@ MPCF_HD float sqrt_rn(const float x)
 // zero, subnormal, infinite or NaN
 MPCF_HD bool not_normal(const float x) { return __builtin_amdgcn_classf(x, 0x2f7); }
 MPCF_HD bool not_normal(const double x) { return __builtin_amdgcn_class(x, 0x2f7); }
-MPCF_HD bool any_lane(const bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; }
+MPCF_HD bool any_lane(const bool b, const uint64_t lanes = ~uint64_t(0)) { return (__builtin_amdgcn_ballot_w64(b) & lanes) != 0; }
 #else
 template <typename T> constexpr bool kQuick = false;
 template <typename T> MPCF_HD T rcp_rn(const T b) { return T(1.0) / b; }
 template <typename T> MPCF_HD T div_rn(const T a, const T b, const T) { return a / b; }
 template <typename T> MPCF_HD T sqrt_rn(const T x) { return msqrt(x); }
 template <typename T> MPCF_HD bool not_normal(const T) { return false; }
-MPCF_HD bool any_lane(const bool b) { return b; }
+MPCF_HD bool any_lane(const bool b, const uint64_t = ~uint64_t(0)) { return b; }
 #endif
 
 // SYNC: the workgroup's waves meet here.  Nothing is exchanged: the barrier
@@ -593,13 +593,16 @@ MPCF_HD FaceFluxT<T> riemann_as(const PrimT<T> L, const PrimT<T> Rt, bool* odd)
     return o;
 }
 
-template <int D, typename T, bool FAST, bool SYNC = false>
-MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt)
+// LANES: the lanes of the wave whose faces are used, the only ones whose operands
+// count; again (a test hook's): set where the wave solved its faces twice
+template <int D, typename T, bool FAST, bool SYNC = false, uint64_t LANES = ~uint64_t(0)>
+MPCF_HD FaceFluxT<T> riemann(const PrimT<T> L, const PrimT<T> Rt, bool* again = nullptr)
 {
     if constexpr (!FAST && kQuick<T> && sizeof(T) == 4) {
         bool odd = false;
         FaceFluxT<T> o = riemann_as<D, T, FAST, SYNC, true>(L, Rt, &odd);
-        if (__builtin_expect(any_lane(odd), 0)) o = riemann_as<D, T, FAST, false, false>(L, Rt, nullptr);
+        if (again) *again = any_lane(odd, LANES);
+        if (__builtin_expect(any_lane(odd, LANES), 0)) o = riemann_as<D, T, FAST, false, false>(L, Rt, nullptr);
         return o;
     } else {
         return riemann_as<D, T, FAST, SYNC, false>(L, Rt, nullptr);

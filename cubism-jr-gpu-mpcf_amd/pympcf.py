@@ -33,7 +33,7 @@ EXPORTS = [
     "mpcf_last_error", "mpcf_version", "mpcf_create", "mpcf_destroy", "mpcf_set_pipeline", "mpcf_set_stream",
     "mpcf_get_stream", "mpcf_set_bc", "mpcf_upload", "mpcf_download", "mpcf_load_ghosts",
     "mpcf_max_sos", "mpcf_convection", "mpcf_update", "mpcf_process_all", "mpcf_step",
-    "mpcf_last_dt", "mpcf_synchronize", "mpcf_query", "mpcf_test_weno", "mpcf_test_face",
+    "mpcf_last_dt", "mpcf_synchronize", "mpcf_query", "mpcf_test_weno", "mpcf_test_face", "mpcf_test_rows",
     "mpcf_timing_enable", "mpcf_timing_read", "mpcf_ic_shock_tube", "mpcf_ic_shock_bubble",
     "mpcf_ic_bubble_cloud", "mpcf_ic_bubble_collapse", "mpcf_flop_count", "mpcf_host_weno",
     "mpcf_host_face", "mpcf_case_bytes", "mpcf_batch_create", "mpcf_batch_destroy", "mpcf_batch_add",
@@ -127,6 +127,7 @@ def lib():
         L.mpcf_query.argtypes = [P, P]
         L.mpcf_test_weno.argtypes = [I, P, P, P, C.c_uint]
         L.mpcf_test_face.argtypes = [I, I, P, P, C.c_uint]
+        L.mpcf_test_rows.argtypes = [I, P, P, C.c_uint]
         L.mpcf_flop_count.argtypes = [C.c_uint, P]
         L.mpcf_host_weno.argtypes = [I, P, P, P, C.c_uint]
         L.mpcf_host_face.argtypes = [I, I, P, P, C.c_uint]
@@ -507,6 +508,14 @@ def test_face(st, d, fast=False, p64=False):
     out = np.empty((n, 12), np.float32)
     flags = (FLAG_FAST if fast or p64 else 0) | (FLAG_P64 if p64 else 0)
     _check(lib().mpcf_test_face(n, d, _ptr(s), _ptr(out), flags))
+    return out
+
+
+def test_rows(st, fast=False):
+    s = np.ascontiguousarray(st, dtype=np.float32)
+    assert s.shape[1:] == (7, 68), s.shape
+    out = np.empty(s.shape[0], np.int32)
+    _check(lib().mpcf_test_rows(s.shape[0], _ptr(s), _ptr(out), FLAG_FAST if fast else 0))
     return out
 
 

@@ -562,9 +562,15 @@ int mpcf_host_face(int n, int dir, const float* st, float* out, unsigned flags);
  *     (GPUonly.cuh:177-194).
  *   mpcf_test_face: st = n x 7 x 6 conserved values at the stencil points
  *     i-3..i+2 of face i-1/2 in direction dir; out = n x 12: the seven fluxes,
- *     the HLLC face velocity, Gm, Gp, Pm, Pp (GPUkernels.cu:203-287). */
+ *     the HLLC face velocity, Gm, Gp, Pm, Pp (GPUkernels.cu:203-287).
+ *   mpcf_test_rows: st = n x 7 x 68 conserved values, each row the cells of a
+ *     wave of the x+y sweep (64, and two beside them on either side); again[i]:
+ *     whether the bit-exact build evaluates that wave's windows (bit 0) or
+ *     faces (bit 1) a second time, with the IEEE quotients, because an operand
+ *     is beyond the quick ones' range (FAST builds: never). */
 int mpcf_test_weno(int n, const float* in5, float* minus, float* plus, unsigned flags);
 int mpcf_test_face(int n, int dir, const float* st, float* out, unsigned flags);
+int mpcf_test_rows(int n, const float* st, int* again, unsigned flags);
 
 /* ------------------------------------------------------------------------
  * Serving: a stream of independent requests advanced with continuous
