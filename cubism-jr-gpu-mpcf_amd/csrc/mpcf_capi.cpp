@@ -599,6 +599,9 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
         return MPCF_OK;
     };
     if (n < (size_t(1) << 18)) return pageable();
+    // what the stream still has to do is waited for before the chunks are taken:
+    // a transfer behind a long run of steps holds up no other stream's
+    HIP_TRY(hipStreamSynchronize(s));
     PinnedChunks& P = pinned_chunks();
     std::lock_guard<std::mutex> lk(P.mu);
     // at least four chunks, so that the two copies of most of them overlap
