@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -445,9 +446,10 @@ namespace {
 // (binary32 or binary64) and the storage type on the device
 // Transfers from and into pageable host memory: the runtime's own path moves
 // 7 to 30 GB/s, a copy from or into pinned memory about 55 GB/s.  Transfers of
-// 256 KB or more go through one process-wide pair of pinned chunks
+// 256 KB or more go through a pair of pinned chunks of the stream's device
 // (allocated on first use, kept for the life of the process; one transfer at a
-// time): the copy engine fills or empties one chunk while host threads move
+// time and device, as the events only serve streams of the device they were
+// created on): the copy engine fills or empties one chunk while host threads move
 // the other out of or into the caller's arrays.
 struct PinnedChunks
 {
@@ -457,10 +459,13 @@ struct PinnedChunks
     size_t cap = 0;
 };
 
-PinnedChunks& pinned_chunks()
+PinnedChunks& pinned_chunks(const int device)
 {
-    static PinnedChunks p;
-    return p;
+    // never destroyed: a copy may be running when the process ends
+    static std::mutex& mu = *new std::mutex();
+    static std::map<int, PinnedChunks>& all = *new std::map<int, PinnedChunks>();
+    std::lock_guard<std::mutex> lk(mu);
+    return all[device];
 }
 
 // A host copy of `n` bytes in pieces move(offset, length), split over a pool of
@@ -546,20 +551,23 @@ void mpcf::detail::parallel_copy(void* dst, const void* src, const size_t n)
 
 namespace {
 
-// pinned chunks of at least `want` bytes (at most kChunkMax), allocated; the
-// caller holds P.mu.  Small transfers get along with small chunks: pinning
+// pinned chunks and events of `device` for at least `want` bytes (at most
+// kChunkMax), allocated; the caller holds P.mu.  Small transfers get along with small chunks: pinning
 // 128 MB costs more than they do.  false: the host has no such memory left
 constexpr size_t kChunkMin = size_t(4) << 20, kChunkMax = size_t(64) << 20;
-bool ready_chunks(PinnedChunks& P, const size_t want)
+bool ready_chunks(PinnedChunks& P, const int device, const size_t want)
 {
     if (P.cap >= want) return true;
     const size_t cap = want <= kChunkMin ? kChunkMin : kChunkMax;
     char* b[2] = {nullptr, nullptr};
-    hipError_t e = hipSuccess;
+    int current = device;   // the caller's, which may be another than the stream's
+    hipError_t e = hipGetDevice(&current);
+    if (e == hipSuccess && current != device) e = hipSetDevice(device);
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
         if (!P.ev[i]) e = hipEventCreateWithFlags(&P.ev[i], hipEventDisableTiming);
         if (e == hipSuccess) e = hipHostMalloc((void**)&b[i], cap, hipHostMallocDefault);
     }
+    if (current != device) (void)hipSetDevice(current);
     if (e != hipSuccess) {
         for (int i = 0; i < 2; ++i)
             if (b[i]) hipHostFree(b[i]);
@@ -602,11 +610,14 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
     // what the stream still has to do is waited for before the chunks are taken:
     // a transfer behind a long run of steps holds up no other stream's
     HIP_TRY(hipStreamSynchronize(s));
-    PinnedChunks& P = pinned_chunks();
+    int device = 0;
+    if (s) HIP_TRY(hipStreamGetDevice(s, &device));
+    else   HIP_TRY(hipGetDevice(&device));
+    PinnedChunks& P = pinned_chunks(device);
     std::lock_guard<std::mutex> lk(P.mu);
     // at least four chunks, so that the two copies of most of them overlap
     const size_t cap = std::min(kChunkMax, std::max(size_t(1) << 20, (n / 4 + 4095) / 4096 * 4096));
-    if (!ready_chunks(P, cap)) return pageable();   // no pinned memory to be had
+    if (!ready_chunks(P, device, cap)) return pageable();   // no pinned memory to be had
     const size_t nchunk = (n + cap - 1) / cap;
     auto length = [&](const size_t k) { return std::min(cap, n - k * cap); };
     // chunk k of the host arrays <-> its pinned buffer, by the pool of threads

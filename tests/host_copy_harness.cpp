@@ -145,6 +145,18 @@ bool busy()
     return first && same && rc0 == MPCF_OK && host == dev;
 }
 
+// contexts on two devices, the current device not always the stream's
+bool devices()
+{
+    Stream s[2];
+    s[1].device = 1;
+    for (int k = 0; k < 6; ++k) {
+        device = k & 1;
+        if (!round_trip(s[(k >> 1) & 1], 7, 100000 + 900000 * k, k) || device != (k & 1)) return false;
+    }
+    return pinned > 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -152,6 +164,7 @@ int main(int argc, char** argv)
     const std::string mode = argc > 1 ? argv[1] : "";
     bool ok = false;
     if (mode == "busy") ok = busy();
+    if (mode == "devices") ok = devices();
     std::printf("%s %s\n", mode.c_str(), ok ? "ok" : "failed");
     std::fflush(stdout);
     std::_Exit(ok ? 0 : 1);   // the library's copy threads live as long as the process

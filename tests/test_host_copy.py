@@ -31,3 +31,7 @@ def run(harness, mode):
 
 def test_a_busy_stream_does_not_hold_up_another(harness):
     run(harness, "busy")
+
+
+def test_streams_of_two_devices(harness):
+    run(harness, "devices")
