@@ -20,6 +20,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -532,7 +533,11 @@ CopyPool& copy_pool()
         const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
         const unsigned nw = std::min(7u, hw - 1);
         for (unsigned i = 0; i < nw; ++i) {
-            P->workers.emplace_back([P, i] { P->work(i); });
+            try {
+                P->workers.emplace_back([P, i] { P->work(i); });
+            } catch (const std::system_error&) {
+                break;   // the host gives no more threads: the copies make do with fewer
+            }
             P->workers.back().detach();
         }
         return P;

@@ -3,6 +3,7 @@
 // host memory, with two devices, streams that can be held busy, and refusals.
 //   host_copy_harness MODE   -> exit code 0 if the transfers do what they should
 #include <hip/hip_runtime.h>
+#include <cerrno>
 #include <chrono>
 #include <condition_variable>
 #include <cstdio>
@@ -32,6 +33,7 @@ int waiting = 0;                              // callers inside a wait for a hel
 thread_local int device = 0;
 bool refuse_pinned = false;
 int pinned = 0;
+int threads_left = 1 << 20;                   // threads that the host still gives
 Stream null_stream;
 
 Stream* stream(hipStream_t s) { return s ? (Stream*)s : &null_stream; }
@@ -57,6 +59,12 @@ void release(Stream& s)
 }  // namespace
 
 extern "C" {
+// every thread of the program starts here (the linker wraps the calls)
+int __real_pthread_create(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*);
+int __wrap_pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* x)
+{
+    return threads_left-- > 0 ? __real_pthread_create(t, a, f, x) : EAGAIN;
+}
 hipError_t hipGetDevice(int* d) { *d = device; return hipSuccess; }
 hipError_t hipSetDevice(int d) { device = d; return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) { *d = s ? stream(s)->device : device; return hipSuccess; }
@@ -157,6 +165,17 @@ bool devices()
     return pinned > 0;
 }
 
+// sizes on both sides of the line to plain copies, chunk edges inside arrays,
+// the small chunks growing into the large ones, more than two full chunks
+bool sizes()
+{
+    Stream s;
+    bool ok = true;
+    for (const size_t per : {size_t(37449), size_t(37450), size_t(600001), size_t(3000017), size_t(24000031)})
+        ok = ok && round_trip(s, 7, per, 7);
+    return ok && round_trip(s, 1, (size_t(4) << 20) + 5, 8);
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -165,6 +184,9 @@ int main(int argc, char** argv)
     bool ok = false;
     if (mode == "busy") ok = busy();
     if (mode == "devices") ok = devices();
+    if (mode == "sizes") ok = sizes();
+    if (mode == "refused") { refuse_pinned = true; ok = sizes() && pinned == 0; }
+    if (mode == "threads") { threads_left = std::atoi(argv[2]); ok = sizes(); }
     std::printf("%s %s\n", mode.c_str(), ok ? "ok" : "failed");
     std::fflush(stdout);
     std::_Exit(ok ? 0 : 1);   // the library's copy threads live as long as the process

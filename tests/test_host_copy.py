@@ -20,12 +20,12 @@ def harness(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-w", "-pthread", "-I", ROCM, "-I", csrc,
                     "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host_copy_harness.cpp"),
                     os.path.join(csrc, "mpcf_capi.cpp"), "-o", str(exe), "-static",
-                    "-Wl,--unresolved-symbols=ignore-all"], check=True, timeout=120)
+                    "-Wl,--unresolved-symbols=ignore-all", "-Wl,--wrap=pthread_create"], check=True, timeout=120)
     return str(exe)
 
 
-def run(harness, mode):
-    r = subprocess.run([harness, mode], capture_output=True, text=True, timeout=60)
+def run(harness, *mode):
+    r = subprocess.run([harness, *mode], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
@@ -35,3 +35,17 @@ def test_a_busy_stream_does_not_hold_up_another(harness):
 
 def test_streams_of_two_devices(harness):
     run(harness, "devices")
+
+
+def test_sizes(harness):
+    run(harness, "sizes")
+
+
+def test_no_pinned_memory_left(harness):
+    run(harness, "refused")
+
+
+@pytest.mark.parametrize("threads", ["0", "2"])
+def test_no_threads_left(harness, threads):
+    """a host that gives no or only some of the copy threads"""
+    run(harness, "threads", threads)
