@@ -1124,6 +1124,29 @@ extern "C" int mpcf_test_rows(int n, const float* st, int* again, unsigned flags
     return MPCF_OK;
 }
 
+extern "C" int mpcf_test_quotient(int op, int n, const void* a, const void* b, void* out)
+{
+    const bool needs_a = op == 1 || op == 2, needs_b = op != 2;
+    if (op < 0 || op > 3 || n < 0 || (n > 0 && (!out || (needs_a && !a) || (needs_b && !b))))
+        return fail(MPCF_EINVAL, "mpcf_test_quotient: bad argument");
+    if (n == 0) return MPCF_OK;
+    const size_t bytes = (size_t)n * (op == 3 ? sizeof(double) : sizeof(float));
+    DevBuf da, db, o;
+    HIP_TRY(hipMalloc(&o.p, bytes));
+    if (needs_a) {
+        HIP_TRY(hipMalloc(&da.p, bytes));
+        HIP_TRY(hipMemcpy(da.p, a, bytes, hipMemcpyHostToDevice));
+    }
+    if (needs_b) {
+        HIP_TRY(hipMalloc(&db.p, bytes));
+        HIP_TRY(hipMemcpy(db.p, b, bytes, hipMemcpyHostToDevice));
+    }
+    mpcf::parity::launch_test_quotient(op, n, da.p, db.p, o.p, nullptr);
+    LAUNCH_CHECK("test_quotient");
+    HIP_TRY(hipMemcpy(out, o.p, bytes, hipMemcpyDeviceToHost));
+    return MPCF_OK;
+}
+
 // ===========================================================================
 // Batched ensembles (mpcf_batch_*): many independent cases of uneven sizes
 // advanced together, one launch per kernel kind per stage, per-case dt on the

@@ -1574,6 +1574,20 @@ __global__ void k_test_rows(const Real* __restrict__ st, int* __restrict__ again
     if (lane == 0) again[blockIdx.x] = (windows ? 1 : 0) | (faces ? 2 : 0);
 }
 
+#if !MPCF_FAST && !MPCF_F64
+// the quick operations by themselves (mpcf_scheme.h): OP 0 rcp_rn(b), 1
+// div_rn(a, b), 2 sqrt_rn(a), all binary32, 3 rcp_rn(b) in binary64
+template <int OP, typename V>
+__global__ void k_test_quotient(const int n, const V* __restrict__ a, const V* __restrict__ b, V* __restrict__ out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    if constexpr (OP == 1)      out[i] = div_rn(a[i], b[i], rcp_rn(b[i]));
+    else if constexpr (OP == 2) out[i] = sqrt_rn(a[i]);
+    else                        out[i] = rcp_rn(b[i]);
+}
+#endif
+
 // ---------------------------------------------------------------------------
 // batched ensemble: one launch per kernel kind advances every live case.  A
 // flat block index is mapped to (case, local block) by a binary search over
@@ -2030,6 +2044,18 @@ void launch_test_weno(const int n, const void* in5v, void* mv, void* pv, hipStre
     Real* p = (Real*)pv;
     hipLaunchKernelGGL(k_test_weno, dim3((n + 255) / 256), dim3(256), 0, s, n, in5, m, p);
 }
+
+#if !MPCF_FAST && !MPCF_F64
+void launch_test_quotient(const int op, const int n, const void* a, const void* b, void* out, hipStream_t s)
+{
+    const dim3 grid((n + 255) / 256), block(256);
+    const float *af = (const float*)a, *bf = (const float*)b;
+    if (op == 0)      hipLaunchKernelGGL((k_test_quotient<0, float>), grid, block, 0, s, n, af, bf, (float*)out);
+    else if (op == 1) hipLaunchKernelGGL((k_test_quotient<1, float>), grid, block, 0, s, n, af, bf, (float*)out);
+    else if (op == 2) hipLaunchKernelGGL((k_test_quotient<2, float>), grid, block, 0, s, n, af, bf, (float*)out);
+    else hipLaunchKernelGGL((k_test_quotient<3, double>), grid, block, 0, s, n, (const double*)a, (const double*)b, (double*)out);
+}
+#endif
 
 void launch_test_rows(const int n, const void* st, int* again, hipStream_t s)
 {

@@ -128,6 +128,9 @@ int whole_chunk(const Geom& g, int dir);                                        
 } }
 
 MPCF_DECLARE_LAUNCHERS(parity)
+namespace mpcf { namespace parity {
+void launch_test_quotient(int op, int n, const void* a, const void* b, void* out, hipStream_t s);
+} }
 MPCF_DECLARE_LAUNCHERS(fast)
 MPCF_DECLARE_LAUNCHERS(fastp)
 MPCF_DECLARE_LAUNCHERS(fastpe)

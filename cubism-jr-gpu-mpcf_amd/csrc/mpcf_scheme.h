@@ -113,20 +113,20 @@ template <bool FAST, typename T> MPCF_HD T qsqrt(const T a) { return FAST ? msqr
 // scale and repair extreme operands (f32 quotient 6 instructions, not 11, of
 // which 4 run at half rate; square root 5, not 14; f64 reciprocal 6, not 11).
 // The callers check the range and fall back to the IEEE operation.
+// mpcf_test_quotient runs them by themselves, on every operand named here:
 //  * rcp_rn(float): one Newton step from v_rcp_f32 gives the correctly rounded
-//    reciprocal of each of the 2^23 significands (all of them tried on the
-//    device).
+//    reciprocal of each of the 2^23 significands.
 //  * div_rn: with a correctly rounded reciprocal one residual correction of
 //    a*y rounds correctly.  The error before the last rounding is below 2.25
 //    2^-24 units in the last place, so only quotients that close to a rounding
-//    midpoint could fail; these are the 2.7e8 significand pairs with
-//    |2^24 a - m b| or |2^25 a - m b| <= 24, all of which were tried.
-//  * sqrt_rn: all 2^24 significands and exponent parities were tried.
+//    midpoint could fail: |2^24 a - m b| < 4.5 for an odd m (quotients from 1;
+//    2^25 below 1).  The 2.9e7 pairs of significands with residues of at most 5
+//    all round correctly.
+//  * sqrt_rn: so do all 2^24 significands and exponent parities.
 //  * rcp_rn(double): a cubic step from v_rcp_f64 (2^-24.3) is within one unit
 //    in the last place, and Markstein's last step y + y (1 - b y) then rounds
-//    correctly (unless b's significand is all ones, which 10 i^2 of a binary32
-//    i never is; 4.3e9 random b and the 65536 significands below all ones
-//    were tried).
+//    correctly, but for a significand of all ones, which that does not cover:
+//    v_rcp_f64's value for it leads to the right result.
 #if defined(__HIP_DEVICE_COMPILE__)
 template <typename T> constexpr bool kQuick = std::is_floating_point<T>::value;
 MPCF_HD float rcp_rn(const float b)

@@ -34,6 +34,7 @@ EXPORTS = [
     "mpcf_get_stream", "mpcf_set_bc", "mpcf_upload", "mpcf_download", "mpcf_load_ghosts",
     "mpcf_max_sos", "mpcf_convection", "mpcf_update", "mpcf_process_all", "mpcf_step",
     "mpcf_last_dt", "mpcf_synchronize", "mpcf_query", "mpcf_test_weno", "mpcf_test_face", "mpcf_test_rows",
+    "mpcf_test_quotient",
     "mpcf_timing_enable", "mpcf_timing_read", "mpcf_ic_shock_tube", "mpcf_ic_shock_bubble",
     "mpcf_ic_bubble_cloud", "mpcf_ic_bubble_collapse", "mpcf_flop_count", "mpcf_host_weno",
     "mpcf_host_face", "mpcf_case_bytes", "mpcf_batch_create", "mpcf_batch_destroy", "mpcf_batch_add",
@@ -128,6 +129,7 @@ def lib():
         L.mpcf_test_weno.argtypes = [I, P, P, P, C.c_uint]
         L.mpcf_test_face.argtypes = [I, I, P, P, C.c_uint]
         L.mpcf_test_rows.argtypes = [I, P, P, C.c_uint]
+        L.mpcf_test_quotient.argtypes = [I, I, P, P, P]
         L.mpcf_flop_count.argtypes = [C.c_uint, P]
         L.mpcf_host_weno.argtypes = [I, P, P, P, C.c_uint]
         L.mpcf_host_face.argtypes = [I, I, P, P, C.c_uint]
@@ -516,6 +518,19 @@ def test_rows(st, fast=False):
     assert s.shape[1:] == (7, 68), s.shape
     out = np.empty(s.shape[0], np.int32)
     _check(lib().mpcf_test_rows(s.shape[0], _ptr(s), _ptr(out), FLAG_FAST if fast else 0))
+    return out
+
+
+def test_quotient(op, a=None, b=None):
+    """the bit-exact build's quick operations: "rcp" 1/b, "div" a/b, "sqrt" of a
+    (binary32), "rcp64" 1/b (binary64)"""
+    k = ("rcp", "div", "sqrt", "rcp64").index(op)
+    dt = np.float64 if k == 3 else np.float32
+    a, b = (None if x is None else np.ascontiguousarray(x, dtype=dt) for x in (a, b))
+    n = (a if b is None else b).shape[0]
+    assert all(x is None or x.shape == (n,) for x in (a, b))
+    out = np.empty(n, dt)
+    _check(lib().mpcf_test_quotient(k, n, None if a is None else _ptr(a), None if b is None else _ptr(b), _ptr(out)))
     return out
 
 

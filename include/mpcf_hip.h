@@ -567,10 +567,14 @@ int mpcf_host_face(int n, int dir, const float* st, float* out, unsigned flags);
  *     wave of the x+y sweep (64, and two beside them on either side); again[i]:
  *     whether the bit-exact build evaluates that wave's windows (bit 0) or
  *     faces (bit 1) a second time, with the IEEE quotients, because an operand
- *     is beyond the quick ones' range (FAST builds: never). */
+ *     is beyond the quick ones' range (FAST builds: never).
+ *   mpcf_test_quotient: the quick operations by themselves, of operands in their
+ *     range: op 0 out = 1 / b, 1 out = a / b, 2 out = sqrt(a), all binary32, 3
+ *     out = 1 / b in binary64 (the operand that op does not take may be NULL). */
 int mpcf_test_weno(int n, const float* in5, float* minus, float* plus, unsigned flags);
 int mpcf_test_face(int n, int dir, const float* st, float* out, unsigned flags);
 int mpcf_test_rows(int n, const float* st, int* again, unsigned flags);
+int mpcf_test_quotient(int op, int n, const void* a, const void* b, void* out);
 
 /* ------------------------------------------------------------------------
  * Serving: a stream of independent requests advanced with continuous
