@@ -594,7 +594,14 @@ __device__ __forceinline__ SosT sweep_yz_column(const Geom& g, const StageArgs& 
             for (int f = 0; f < NU; ++f) ein.u[f] = r0[f];                   // cell k-1
         }
         m.push(q);
+        // The stages' z sweeps of the P64 builds, whose folded speed of sound is
+        // binary64, take 257 to 260 VGPRs and run one wave per SIMD unless a
+        // row's instructions keep out of the next row's (246 to 253 VGPRs): z
+        // sweep of 128^3 63.1 -> 55.2 us, 192^3 180.6 -> 157.1, E pair 65.7 ->
+        // 57.8 and 189.4 -> 167.3
+        if constexpr (kEPair && is_stage(MODE)) __builtin_amdgcn_sched_barrier(0);
         m.step(A, dtinvh, FLUX, EMIT, E, off(k - 1), ein);
+        if constexpr (kP64 && is_stage(MODE)) __builtin_amdgcn_sched_barrier(0);
         ein = ein_next;
     };
     if constexpr (kUnrollMarch) {
