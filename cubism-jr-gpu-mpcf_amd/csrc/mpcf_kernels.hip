@@ -1815,7 +1815,12 @@ static int pick_chunk(const int nd, const int64_t columns)
 // (four waves per SIMD and more) left small blocks to a few dozen waves
 // marching 16 rows each: FAST x+y / z sweep 42 / 27 us at 32^3, 45 / 29 at
 // 64^3 and 100 / 54 at 128^3, against 9 / 10, 22 / 17 and 96 / 53 here.
-static int whole_march(const int nd, const int64_t blocks, const int dir)
+// lone: one wave holds the x+y sweep's columns.  The workgroup's other three waves
+// leave at once, and three such workgroups run on a CU side by side (one in
+// the binary64 build, whose waves take a whole SIMD): us for (5, ny, 5) counted as
+// above / so, FAST 300 10.8 / 9.5, 3000 22.8 / 18.9, 9000 48.6 / 38.3, 20000
+// 97.3 / 75.7; bit-exact 22.5 / 17.2, 48.1 / 36.7, 117 / 82, 242 / 169.
+static int whole_march(const int nd, const int64_t blocks, const int dir, const bool lone = false)
 {
     const double lat = dir == 3 ? 3.0 : 1.0;
     const double ov = dir == 3 ? 1.0 : kFast ? 3.0 : 2.0;
@@ -1823,9 +1828,9 @@ static int whole_march(const int nd, const int64_t blocks, const int dir)
     double least = 0.0;
     for (int L = nd; L >= 1;) {
         const int nch = (nd + L - 1) / L;
-        const int64_t n = (blocks * nch + 255) / 256;
+        const int64_t n = lone ? (nch + 767) / 768 : (blocks * nch + 255) / 256;
         if (L < nd && n > 64) break;     // the tail no longer matters
-        const double t = lat + (n == 1 ? 1.2 : (double)n) * (L + ov);
+        const double t = lat + (n == 1 && !lone ? 1.2 : (double)n) * (L + ov);
         if (L == nd || t < least) { least = t; best = L; }
         const int next = (nd + nch) / (nch + 1);   // the longest march with more chunks
         L = next < L ? next : L - 1;
@@ -1884,11 +1889,9 @@ static int z_width(const Geom& g) { return z_width(g.nx, (long long)g.nx * g.ny 
 
 // four-wave workgroups of one chunk of the x+y sweep over nz planes / of the
 // z sweep's flattened (x, y) columns, `width` of them a row
-static int xy_blocks(const Geom& g, const int nz)
-{
-    const int waves = ((g.nx + 6) * nz + XY_TILE - 1) / XY_TILE;
-    return (waves + 3) / 4;
-}
+static int xy_waves(const Geom& g, const int nz) { return ((g.nx + 6) * nz + XY_TILE - 1) / XY_TILE; }
+static int xy_blocks(const Geom& g, const int nz) { return (xy_waves(g, nz) + 3) / 4; }
+static bool xy_lone(const Geom& g, const int nz) { return !MPCF_F64 && xy_waves(g, nz) == 1; }
 static int z_blocks(const Geom& g, const int width) { return (width * g.ny + 255) / 256; }
 
 static int rows_grid(const Geom& g)
@@ -1968,7 +1971,7 @@ void launch_sweep(const Geom& g, const int dir, const SweepParams& p, const int 
     const bool whole = A.z0 == 0 && A.z1 == g.nz;   // not a slab
     if (dir == 3) {
         const int nb = xy_blocks(g, nzr);
-        const int chunk = whole ? whole_march(g.ny, nb, 3) : p.fit ? slab_march(g.ny, nb, 3)
+        const int chunk = whole ? whole_march(g.ny, nb, 3, xy_lone(g, nzr)) : p.fit ? slab_march(g.ny, nb, 3)
                                                                             : pick_chunk(g.ny, (int64_t)g.nx * nzr);
         const dim3 grid(nb, (g.ny + chunk - 1) / chunk);
         // a first stage of a folded build does not read R
@@ -2082,7 +2085,8 @@ void launch_test_face(const int n, const int dir, const void* stv, void* outv, h
 // the march length of a whole-block x+y (dir 3) or z (dir 2) launch that runs alone
 int whole_chunk(const Geom& g, const int dir)
 {
-    return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3) : whole_march(g.nz, z_blocks(g, z_width(g)), 2);
+    return dir == 3 ? whole_march(g.ny, xy_blocks(g, g.nz), 3, xy_lone(g, g.nz))
+                    : whole_march(g.nz, z_blocks(g, z_width(g)), 2);
 }
 
 // positions a wave of the fused x+y sweep stores
