@@ -1874,15 +1874,19 @@ static int slab_march(const int nd, const int64_t blocks, const int dir)
 // rounded up to 32 columns give every half wave one whole 128-byte line a
 // field, where the packed columns of an odd nx read and write each line in
 // parts, from two waves.  Smaller blocks stay in the L2s and only feel the idle
-// lanes, and the EPAIR build (eight fields and more arithmetic) gains later.  Measured,
-// packed / rounded z sweep, us: 80^3 22.2 / 23.8, 90^3 28.2 / 26.4, 129x64x64
-// 24.7 / 23.6, 97^3 37.5 / 34.6, 161^3 126 / 103, 193^3 234 / 185; EPAIR
-// 97x120x120 54.8 / 58.6, 129^3 80.0 / 80.0, 50x300x200 107 / 115, 161^3 137 /
-// 129, 193^3 245 / 204.  The bit-exact and binary64 sweeps are bound by their
+// lanes, and so do rows of up to 48 columns, most of whose lanes may idle, until
+// the padded rows fill some 8 M elements a field; of those, rows of whole
+// 64-byte halves of a line never gain.  Time of the rounded against the packed z
+// sweep: below 2^19 cells 0.99-1.20; nx 56-161, 0.6 to 4 M cells, 0.75-1.07
+// (161^3 126 / 103 us, 193^3 234 / 185); nx 5-44 below 15 2^19 padded elements
+// 0.95-1.18, above 0.81-1.01; nx 16 and 48 0.95-1.21.  Alike in the P64 and
+// E-pair builds.  The bit-exact and binary64 sweeps are bound by their
 // arithmetic and lose what the idle lanes cost (193^3 335 / 373)
 int z_width(const int nx, const long long cells)
 {
-    if (!kFast || cells < (kEPair ? 3LL << 20 : 1LL << 19)) return nx;
+    if (!kFast || cells < 1LL << 19) return nx;
+    const long long padded = cells / nx * ((nx + XOFF + GHOST + 31) / 32 * 32);
+    if (nx <= 48 && (nx % 16 == 0 || padded < 15LL << 19)) return nx;
     return (nx + 31) / 32 * 32;
 }
 static int z_width(const Geom& g) { return z_width(g.nx, (long long)g.nx * g.ny * g.nz); }
