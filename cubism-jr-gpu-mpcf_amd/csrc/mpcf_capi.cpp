@@ -593,8 +593,8 @@ bool ready_chunks(PinnedChunks& P, const int device, const size_t want)
 // ordered on stream s.  A download is complete on return; an upload has read
 // the host arrays, and its last copies may still run on s.
 // Measured (seven fields, upload / download) against pageable uploads and
-// downloads one field at a time: 0.9 MB 0.09 / 0.10 ms against 0.38 / 0.20,
-// 7 MB 0.26 / 0.29 against 0.30 / 0.64, 470 MB 9.2 / 11.7 against 16.3 / 16.9,
+// downloads one field at a time: 0.9 MB 0.08 / 0.08 ms against 0.16 / 0.20,
+// 7 MB 0.21 / 0.22 against 0.29 / 0.57, 470 MB 9.1 / 10.6 against 15.8 / 15.7,
 // 3.8 GB 69 / 75 against 126 / 84.
 int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const int nh, const size_t per,
                             const bool to_device)
@@ -611,7 +611,12 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
         }
         return MPCF_OK;
     };
-    if (n < (size_t(1) << 18)) return pageable();
+    // one array of up to 4 MB, or 1 MB downloaded: the runtime's own copy takes less
+    // time than the chunks' two (us against through the chunks: up 0.3 MB 31 / 41,
+    // 0.9 MB 52 / 73, 1.3 MB 70 / 92, 3.1 MB 113 / 124, but 4.9 MB 163 / 157; down
+    // 0.3 MB 37 / 45, 0.9 MB 63 / 77, but 1.3 MB 97 / 86)
+    const size_t alone = size_t(to_device ? 4 : 1) << 20;
+    if (n < (size_t(1) << 18) || (nh == 1 && n <= alone)) return pageable();
     // what the stream still has to do is waited for before the chunks are taken:
     // a transfer behind a long run of steps holds up no other stream's
     HIP_TRY(hipStreamSynchronize(s));
@@ -620,8 +625,10 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
     else   HIP_TRY(hipGetDevice(&device));
     PinnedChunks& P = pinned_chunks(device);
     std::lock_guard<std::mutex> lk(P.mu);
-    // at least four chunks, so that the two copies of most of them overlap
-    const size_t cap = std::min(kChunkMax, std::max(size_t(1) << 20, (n / 4 + 4095) / 4096 * 4096));
+    // at least four chunks, so that the two copies of most of them overlap, or two
+    // of up to 4 MB (four of 7.3 MB 240 us, two 205; eight 290)
+    const size_t want = std::max(n / 4, std::min(n / 2, kChunkMin));
+    const size_t cap = std::min(kChunkMax, std::max(size_t(1) << 20, (want + 4095) / 4096 * 4096));
     if (!ready_chunks(P, device, cap)) return pageable();   // no pinned memory to be had
     const size_t nchunk = (n + cap - 1) / cap;
     auto length = [&](const size_t k) { return std::min(cap, n - k * cap); };

@@ -173,7 +173,23 @@ bool sizes()
     bool ok = true;
     for (const size_t per : {size_t(37449), size_t(37450), size_t(600001), size_t(3000017), size_t(24000031)})
         ok = ok && round_trip(s, 7, per, 7);
-    return ok && round_trip(s, 1, (size_t(4) << 20) + 5, 8);
+    for (const size_t n : {(size_t(1) << 20), (size_t(1) << 20) + 1, (size_t(4) << 20), (size_t(4) << 20) + 5})
+        ok = ok && round_trip(s, 1, n, 8);
+    return ok;
+}
+
+// one array of up to 4 MB, or 1 MB downloaded, goes to the runtime as it is
+bool single()
+{
+    Stream s;
+    std::vector<char> host(4 << 20, 'h'), dev(4 << 20, 'd');
+    void* h = host.data();
+    bool ok = mpcf::detail::host_copy((hipStream_t)&s, dev.data(), &h, 1, dev.size(), true) == MPCF_OK && host == dev;
+    host.assign(1 << 20, 'x');
+    h = host.data();
+    ok = ok && mpcf::detail::host_copy((hipStream_t)&s, dev.data(), &h, 1, host.size(), false) == MPCF_OK &&
+         std::memcmp(host.data(), dev.data(), host.size()) == 0;
+    return ok && pinned == 0;
 }
 
 }  // namespace
@@ -185,6 +201,7 @@ int main(int argc, char** argv)
     if (mode == "busy") ok = busy();
     if (mode == "devices") ok = devices();
     if (mode == "sizes") ok = sizes();
+    if (mode == "single") ok = single();
     if (mode == "refused") { refuse_pinned = true; ok = sizes() && pinned == 0; }
     if (mode == "threads") { threads_left = std::atoi(argv[2]); ok = sizes(); }
     std::printf("%s %s\n", mode.c_str(), ok ? "ok" : "failed");

@@ -41,6 +41,10 @@ def test_sizes(harness):
     run(harness, "sizes")
 
 
+def test_one_array_of_a_few_mb(harness):
+    run(harness, "single")
+
+
 def test_no_pinned_memory_left(harness):
     run(harness, "refused")
 
