@@ -442,9 +442,6 @@ extern "C" int mpcf_halo_import(mpcf_ctx* c, int face, const void* src)
 
 namespace {
 
-// host fields <-> the padded device layout, one field at a time through the
-// accumulator area (free between stages), converting between the host type
-// (binary32 or binary64) and the storage type on the device
 // Transfers from and into pageable host memory: the runtime's own path moves
 // 7 to 30 GB/s, a copy from or into pinned memory about 55 GB/s.  Transfers of
 // 256 KB or more go through a pair of pinned chunks of the stream's device
@@ -686,6 +683,9 @@ int mpcf::detail::host_copy(hipStream_t s, void* devv, void* const* host, const 
 
 namespace {
 
+// host fields <-> the padded device layout, as many at a time as the accumulator
+// area (free between stages) holds, converting between the host type (binary32
+// or binary64) and the storage type on the device
 int transfer(mpcf_ctx* c, const int which, void* const* fields, const int host_f64, const bool to_device,
              const char* what)
 {

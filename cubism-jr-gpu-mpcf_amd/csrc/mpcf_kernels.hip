@@ -882,18 +882,11 @@ __device__ __forceinline__ Prim prim_from_left(const Prim& q)
     o.p = from_left(q.p); o.G = from_left(q.G); o.P = from_left(q.P);
     return o;
 }
-__device__ __forceinline__ Prim prim_from_right(const Prim& q)
-{
-    Prim o;
-    o.r = from_right(q.r); o.u = from_right(q.u); o.v = from_right(q.v); o.w = from_right(q.w);
-    o.p = from_right(q.p); o.G = from_right(q.G); o.P = from_right(q.P);
-    return o;
-}
 
 // workgroups go to the XCDs round-robin by linear id; this maps linear id
 // `lin` of a grid of n to a tile index such that each XCD takes a contiguous
 // run of tiles, so that neighbouring tiles of the fused x+y sweep (which
-// overlap by two positions and share partial cache lines) meet in one L2.
+// overlap by 64 - XY_TILE positions and share partial cache lines) meet in one L2.
 // For grids of equal-cost tiles (one block)
 __device__ __forceinline__ int xcd_order(const int lin, const int n)
 {
@@ -1696,7 +1689,7 @@ void kb_sweep_z(const BatchDev B, const Real a, const Real b, const int fold, co
 // which measured 1.7x slower than flat launches).  Each workgroup pulls items
 // from a device queue (an atomic counter) until it is empty; an item is one
 // workgroup's share of one case's x+y sweep (W = blockDim.x / 64 consecutive
-// 62-position tiles over one y-chunk) or z sweep (blockDim.x columns over one
+// tiles of XY_TILE positions over one y-chunk) or z sweep (blockDim.x columns over one
 // z-chunk), running the single-case bodies, so every case gets exactly the
 // arithmetic it gets alone.  The queue holds the items of the larger cases
 // first, so the small ones fill the launch's tail.
@@ -1862,8 +1855,9 @@ static int slab_march(const int nd, const int64_t blocks, const int dir)
         const int64_t n = (blocks * nch + 255) / 256;
         if (n > nmax && least > 0.0) break;
         const double t = (double)n * (L + ov);
-        if (n < nmin) best = L;            // too few workgroups: shorter marches, down to 8 rows
-        else if (least == 0.0 || t < least) { least = t; best = L; }
+        // fewer than nmin only with the longest marches: a slab of two million
+        // cells or more always reaches it
+        if (n >= nmin && (least == 0.0 || t < least)) { least = t; best = L; }
         const int next = (nd + nch) / (nch + 1);   // the longest march with more chunks
         L = next < L ? next : L - 1;
     }

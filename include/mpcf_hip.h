@@ -263,7 +263,8 @@ int mpcf_query(mpcf_ctx* ctx, long long out[8]);
  * bracketed by HIP events on the context stream (the reference's
  * tCUDA_START/tCUDA_STOP timers, source/GPU/GPU.h:25-35).  mpcf_timing_read
  * synchronizes and returns, per kernel class, the summed milliseconds and the
- * number of launches since the last read:
+ * number of launches since the last read (whole-block steps then take dt in a
+ * launch of its own, class 1, instead of in their first x+y sweep):
  *   0 ghost fill, 1 max speed of sound, 2 dt, 3 x sweep (or the fused x+y
  *   sweep), 4 y sweep (split variant only), 5 z sweep (+ register update),
  *   6 update, 7 other. */
