@@ -129,13 +129,13 @@ int pipeline_slabs(const mpcf_ctx* c)
 {
     if (c->pipe_req >= 0) return c->pipe_req;
     // the split sweeps are all VALU-bound: slabs give them nothing to overlap
-    // (measured on MI355X at 512^3, bit-exact build: whole-block 50.3 ms a
-    // step, 4 slabs 50.5, 8 slabs 51.8)
+    // (measured on MI355X at 512^3, bit-exact build: whole-block 50.0 ms a
+    // step, 4 slabs 50.6, 8 slabs 51.8)
     if (split_xy(c)) return 0;
     // so is the bit-exact binary32 build's fused sweep, whose division and
     // binary64 weight sequences make both sweeps VALU-bound (512^3: whole-
-    // block 48.1 ms a step, 4 slabs 49.4, 8 slabs 49.9; 384^3: whole 20.2,
-    // 3 slabs 20.6, 6 slabs 21.0)
+    // block 46.0 ms a step, 4 slabs 45.6-46.3, 8 slabs 45.7; 384^3: whole 19.3,
+    // 3 slabs 19.7, 6 slabs 19.9)
     if (!(c->flags & MPCF_FLAG_FAST)) return 0;
     // blocks of 2^24 cells or more, slabs by depth as measured on MI355X (fast
     // build, cubes, ms a step): 256^3 4 slabs (2.50; 2.56 with 3, 2.55 whole);

@@ -807,8 +807,9 @@ void k_sweep_x(const Geom g, const StageArgs A, const int chunk)
 // inside the wave and store 58.  The row's edge values cost FAST 14 differences
 // and the registers of the LDS reads against 6.5 % fewer waves: 512^3 19.4 ms a
 // step against 18.8, 256^3 whole-block 2.69 against 2.60; the bit-exact build,
-// with 3 times the arithmetic per cell, gains: 256^3 6.32 against 6.45, a
-// 600x300x6 block 0.545 against 0.565, binary64 128^3 1.42 against 1.43.
+// with 3 times the arithmetic per cell, gains (while it solved its x faces
+// twice): 256^3 6.32 against 6.45, a 600x300x6 block 0.545 against 0.565;
+// binary64 128^3 1.42 against 1.43.
 constexpr bool kHaloLDS = !kFast;
 enum { XY_TILE = kHaloLDS ? 62 : 58 };
 static_assert(!kHaloLDS || !kUnrollXY, "the unrolled march does not refill the rows in LDS");
